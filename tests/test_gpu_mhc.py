@@ -91,3 +91,63 @@ def test_hc_pre_fast_within_tolerance(ctx, oracle, dev):
     for got, want in ((dev.get(yp, hidden), y), (dev.get(qp, hc), post), (dev.get(cp, hc * hc), comb)):
         assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
     print(f"hc_pre 4 x 4096: exact {times[True]:.1f} us, tree sums {times[False]:.1f} us")
+
+
+def _terms(kind, rng, n):
+    """x and a weight row whose products take a sequential f32 sum through
+    the cases of the chunked one."""
+    x = rng.standard_normal(n).astype(np.float32)
+    w = rng.standard_normal(n).astype(np.float32)
+    if kind == "ties":        # few mantissa bits: most additions round a tie
+        x = np.round(x * 4) / 4 + 0.25
+        w = np.exp2(rng.integers(-3, 4, n)) * np.sign(w)
+    elif kind == "range":     # 2^-40 .. 2^40, cancelling pairs
+        w = w * np.exp2(rng.uniform(-40, 40, n))
+        w[1::2] = -w[:n - n % 2:2]
+    elif kind == "zeros":
+        x[rng.random(n) < 0.9] = 0.0
+    elif kind == "huge":      # overflows to infinity part of the way
+        x = x * np.float32(1e19)
+        w = np.abs(w) * np.float32(1e18)
+    return x.astype(np.float32), w.astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties", "range", "zeros", "huge"])
+@pytest.mark.parametrize("hc,hidden", [(1, 31), (1, 1024), (1, 1025), (4, 1024), (4, 1025), (1, 8192), (1, 8193),
+                                       (4, 4096), (4, 4097), (2, 17000)])
+def test_hc_pre_ordered_sums(ctx, oracle, dev, kind, hc, hidden):
+    """The chunked sequential sums at the edges of their chunk sizes and past
+    one segment (16384 terms), bit for bit."""
+    rng = np.random.default_rng(hidden + hc)
+    mix_hc, n = (2 + hc) * hc, hc * hidden
+    x, w0 = _terms(kind, rng, n)
+    fn = np.stack([w0] + [_terms(kind, rng, n)[1] for _ in range(mix_hc - 1)])
+    scale, base = np.full(3, 1e-3, np.float32), rng.standard_normal(mix_hc).astype(np.float32)
+    yp, qp, cp = dev.empty(hidden * 4), dev.empty(hc * 4), dev.empty(hc * hc * 4)
+    ctx.set_exact_numerics(True)
+    ctx.hc_pre_async(dev.put(fn), dev.put(scale), dev.put(base), hc, hidden, 2, 1e-6, dev.put(x), yp, qp, cp)
+    ctx.synchronize()
+    with np.errstate(all="ignore"):
+        y, _, post, comb, _ = oracle.hc_pre(fn, scale, base, x, hc, hidden, 2, 1e-6)
+    for got, w in zip((dev.get(yp, hidden), dev.get(qp, hc), dev.get(cp, hc * hc)), (y, post, comb)):
+        w = np.asarray(w).reshape(-1)
+        assert np.array_equal(np.isnan(got), np.isnan(w))
+        assert np.array_equal(bits(got)[~np.isnan(w)], bits(w)[~np.isnan(w)])
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties", "range", "zeros"])
+@pytest.mark.parametrize("n", [1, 512, 513, 1024, 1025, 4095, 4096])
+@pytest.mark.parametrize("rows", [1, 16])
+def test_rms_norm_ordered_sum(ctx, oracle, dev, kind, n, rows):
+    """The norm's sequential sum of squares over both workgroup sizes, bit
+    for bit."""
+    rng = np.random.default_rng(n)
+    x = np.stack([_terms(kind, rng, n)[0] * np.float32(1.5 ** r) for r in range(rows)])
+    if kind == "range":
+        x = (x * np.exp2(rng.uniform(-30, 30, x.shape))).astype(np.float32)
+    xp, op = dev.put(x), dev.empty(x.nbytes)
+    ctx.set_exact_numerics(True)
+    ctx.rms_norm_async(xp, op, rows, n)
+    ctx.synchronize()
+    want = np.stack([oracle.rms_norm(r) for r in x])
+    assert np.array_equal(bits(dev.get(op, x.size)), bits(want).reshape(-1))

@@ -2,6 +2,7 @@
 // activation quant-dequant, and the fused routed-expert SwiGLU pipeline.
 // Launch helpers and the C ABI live in wohper_hip.hip.
 #pragma once
+#include "ordered_sum.h"
 #include "wh_device.h"
 
 #ifndef WH_LIBM_TABLES_INCLUDED

@@ -11,9 +11,9 @@
 //
 // The dots and the sum of squares are 16384-term sums.  In the reference's
 // order (each term added to a running f32 sum, E/compute.rs:5026-5038) they
-// are serial chains: k_hc_chains runs each chain on one lane of a wave (the
-// 24 dots and the sum of squares side by side), which is bit-exact and
-// bound by the chain's length.  With exact numerics off, k_hc_partials
+// are serial chains: k_hc_chains gives each one a workgroup, which adds its
+// chunks side by side from guessed starts until they fit together
+// (ordered_sum.h), bit-exact.  With exact numerics off, k_hc_partials
 // spreads the terms over many workgroups and k_hc_finish adds the partial
 // sums in a fixed order: the same value up to rounding, reproducible run to
 // run.  Everything after the sums (sigmoids, Sinkhorn, y, hc_post) is
@@ -60,44 +60,40 @@ __device__ __forceinline__ float wh_hc_wave_sum(float v) {
     return v;
 }
 
-// Serial chains: workgroup c (256 threads) runs chain c < mix_hc (fn row
-// c . x) or, for c = mix_hc, the sum of squares.  The 192 threads of waves
-// 1-3 form the products w * x (each rounded on its own) of a chunk of
-// WH_HC_CHUNK terms into an LDS buffer, their loads for the next chunk in
-// flight meanwhile, while thread 0 adds the previous chunk's products to
-// its running sum in order; two buffers alternate.
-#define WH_HC_CHUNK 768u  // 4 terms per producer thread
-__global__ void __launch_bounds__(256) k_hc_chains(wh_hc_args a0) {
+// Ordered sums: workgroup c (1024 threads) runs chain c < mix_hc (fn row
+// c . x) or, for c = mix_hc, the sum of squares, each product rounded on its
+// own and added in order (ordered_sum.h), segments of kL * kC terms at a time
+// with the sum carried on.  A thread's loads of a segment are all issued
+// before the first product.
+template <int kL, int kC>
+__global__ void __launch_bounds__(1024) k_hc_chains(wh_hc_args a0) {
     const wh_hc_args a = wh_hc_at(a0, blockIdx.z);
-    __shared__ __align__(16) float prod[2][WH_HC_CHUNK];
+    extern __shared__ __align__(16) uint8_t osum_lds[];
+    auto& s = *(wh_osum_lds<kL, kC>*)osum_lds;
+    constexpr uint32_t kSeg = kL * kC, kPer = (kSeg + 1023) / 1024;
     const uint32_t t = threadIdx.x, c = blockIdx.x;
-    const uint32_t n_chunks = (a.hc_dim + WH_HC_CHUNK - 1) / WH_HC_CHUNK;
     const float* row = c < a.mix_hc ? a.fn + (size_t)c * a.hc_dim : a.x;
-    const uint32_t u = t - 64;  // producer index (t >= 64)
-    float w[4], xv[4];
-    auto load = [&](uint32_t k) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t e = k * WH_HC_CHUNK + u + 192 * i;
-            const bool on = k < n_chunks && e < a.hc_dim;
-            xv[i] = on ? a.x[e] : 0.0f;
-            w[i] = on ? row[e] : 0.0f;
-        }
-    };
-    if (t >= 64) load(0);
+    __shared__ float carry;
     float acc = 0.0f;
-    for (uint32_t k = 0; k <= n_chunks; ++k) {
-        if (t >= 64 && k < n_chunks) {
+    for (size_t i0 = 0; i0 < a.hc_dim; i0 += kSeg) {
+        float w[kPer], xv[kPer];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) prod[k & 1][u + 192 * i] = w[i] * xv[i];
-            load(k + 1);
+        for (uint32_t k = 0; k < kPer; ++k) {
+            const size_t i = i0 + t + 1024 * k, ic = i < a.hc_dim ? i : 0u;
+            xv[k] = a.x[ic];
+            w[k] = row[ic];
         }
-        if (t == 0 && k > 0) {
-            const float* src = prod[(k - 1) & 1];
-            const uint32_t len = min(WH_HC_CHUNK, a.hc_dim - (k - 1) * WH_HC_CHUNK);
-            acc = wh_ordered_sum_lds(src, len, acc);
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; ++k) {
+            const uint32_t e = t + 1024 * k;
+            if (e < kSeg) s.rows[wh_osum_at<kL>(e)] = i0 + e < a.hc_dim ? w[k] * xv[k] : -0.0f;
         }
-        __syncthreads();
+        acc = wh_ordered_sum_wg<1024, kL, kC>(s, acc);
+        if (i0 + kSeg < a.hc_dim) {  // the next segment's start, for every wave's guess
+            if (t == 0) carry = acc;
+            __syncthreads();
+            acc = carry;
+        }
     }
     if (t == 0) a.sums[c] = acc;
 }

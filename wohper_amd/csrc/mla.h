@@ -160,17 +160,35 @@ __global__ void __launch_bounds__(kT) k_rowpost(wh_rowpost_args a) {
                 inv_s = 1.0f / sqrtf(r / (float)n + 1.0e-6f);
             }
         } else {
-            // the reference's order: every product rounded on its own in
-            // parallel, then one lane adds them in sequence
-            __shared__ __align__(16) float sq[WH_ROWPOST_MAX];
+            // the reference's order: every product rounded on its own, then
+            // the sequential sum by the whole workgroup (ordered_sum.h); up
+            // to 512 terms one lane adds them: 64 heads of 512 took 7.3 us
+            // that way and 8.6 us with the tables and the check
+            constexpr int kMaxL = WH_ROWPOST_MAX / 32;
+            __shared__ __align__(16) wh_osum_lds<kMaxL, 32> os;
+            auto stage = [&](auto l) {
+                constexpr int kL = decltype(l)::value;
+                auto& s = *(wh_osum_lds<kL, 32>*)&os;
 #pragma unroll
-            for (int k = 0; k < kPer; ++k)
-                if (t + kT * k < n) sq[t + kT * k] = xv[k] * xv[k];
-            __syncthreads();
-            if (t == 0) {
-                const float s = wh_ordered_sum_lds(sq, n, 0.0f);
-                inv_s = 1.0f / sqrtf(s / (float)n + 1.0e-6f);
+                for (int k = 0; k < kPer; ++k) {
+                    const uint32_t i = t + kT * k;
+                    if (i < 32 * kL) s.rows[wh_osum_at<kL>(i)] = i < n ? xv[k] * xv[k] : -0.0f;
+                }
+                return wh_ordered_sum_wg<kT, kL, 32>(s, 0.0f);
+            };
+            float s;
+            if (n <= 512) {
+#pragma unroll
+                for (int k = 0; k < 512 / kT + (kT > 512); ++k)
+                    if (t + kT * k < n) os.rows[t + kT * k] = xv[k] * xv[k];
+                __syncthreads();
+                s = t == 0 ? wh_ordered_sum_lds(os.rows, n, 0.0f) : 0.0f;
+            } else if (n <= 1024) {
+                s = stage(std::integral_constant<int, 32>());
+            } else {
+                s = stage(std::integral_constant<int, kMaxL>());
             }
+            if (t == 0) inv_s = 1.0f / sqrtf(s / (float)n + 1.0e-6f);
         }
         __syncthreads();
         const float inv = inv_s;
