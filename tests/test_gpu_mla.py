@@ -157,6 +157,28 @@ def test_window_attention_bit_exact(ctx, oracle, dev, n_win, n_comp, sink, pos):
     assert np.array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("heads,hd,nope,pairs", [(1, 64, 0, 32), (3, 128, 70, 20), (16, 512, 448, 32),
+                                                 (65, 1024, 960, 32), (4, 512, 512, 0)])
+@pytest.mark.parametrize("n_win,n_comp", [(0, 1), (63, 0), (64, 0), (64, 1), (128, 127), (128, 384), (128, 385),
+                                          (128, 896), (128, 897), (128, 1920)])
+def test_window_attention_shapes_bit_exact(ctx, oracle, dev, heads, hd, nope, pairs, n_win, n_comp):
+    """Head counts and key counts at the edges of the tiles, of the one- and
+    two-launch weights and of the denominator's chunked sum, with keys whose
+    scores spread over the exponential's range."""
+    rng = np.random.default_rng(heads * 7 + n_comp)
+    inv = oracle.rope_inv_freqs(2 * max(pairs, 1), 160000.0, oracle.DEEPSEEK_V4_YARN)
+    q = (rng.standard_normal((heads, hd)) * 3).astype(np.float32)
+    win = rng.standard_normal((n_win, hd)).astype(np.float32)
+    comp = rng.standard_normal((n_comp, hd)).astype(np.float32)
+    sk = rng.standard_normal(heads).astype(np.float32)
+    outp, scp = dev.empty(heads * hd * 4), dev.empty(heads * (n_win + n_comp) * 4)
+    ctx.window_attention_async(dev.put(q), heads, hd, nope, dev.put(win) if n_win else 0, n_win, hd,
+                               dev.put(comp) if n_comp else 0, n_comp, dev.put(sk), dev.put(inv), pairs, 777, scp, outp)
+    ctx.synchronize()
+    want = oracle.window_attention(q, hd, nope, win, comp if n_comp else None, sk, inv[:pairs], 777)
+    assert np.array_equal(bits(dev.get(outp, (heads, hd))), bits(want))
+
+
 # ---------------------------------------------------------------- the layer
 HEADS, NOPE, ROPE, Q_LORA, GROUPS, O_LORA = 64, 448, 64, 1024, 8, 1024
 HEAD_DIM = NOPE + ROPE

@@ -105,6 +105,26 @@ def test_mla_batch_compressed_layer(ctx, oracle, dev):
         ctx.release(h)
 
 
+def test_mla_batch_many_positions(ctx, dev):
+    """35 positions (more than one launch's worth) with key lists from a few
+    rows to 700, so that one launch holds short and long ones: bit for bit the
+    single-token layer's outputs."""
+    L, host, qn, kn, sink, handles = _layer(ctx, dev, 2)
+    cap, ld = 240, HEAD_DIM
+    rng = np.random.default_rng(14)
+    cache0 = (rng.standard_normal((cap, ld)) * 0.3).astype(np.float32)
+    positions = list(range(3, 3 + 18)) + list(range(200, 217))
+    comp = dev.put((rng.standard_normal((700, HEAD_DIM)) * 0.3).astype(np.float32))
+    comps = [(comp, int(k)) for k in rng.integers(1, 701, len(positions))]
+    xs = rng.standard_normal((len(positions), wl.HIDDEN)).astype(np.float32)
+    got, got_cache = _batch(ctx, dev, L, xs, positions, cache0, ld, comps)
+    want, want_cache = _sequential(ctx, dev, L, xs, positions, cache0, ld, comps)
+    assert np.array_equal(bits(got_cache), bits(want_cache))
+    assert np.array_equal(bits(got), bits(want))
+    for h in handles.values():
+        ctx.release(h)
+
+
 def test_mla_batch_order_free_16(ctx, dev):
     """16 positions: with exact numerics the batch equals the single-token
     layer position by position (the decode-once kernels at 16 inputs); with

@@ -246,11 +246,12 @@ struct wh_attn_args {
     uint32_t heads, head_dim, nope_dim, pairs;
     uint32_t n_win, n_comp, win_ld, token_pos;
     float scale;           // head_dim^-0.5 (host powf, as the reference)
-    // a batch of positions (nb > 0): slot z = blockIdx.z takes q and out +
+    // a batch of positions (nb > 0): slot z takes q and out +
     // z * q_ld, scores + z * scores_ld, token_pos = bpos[z], the window of
     // the last wlen cache rows up to that position (win = the cache's row
     // 0), compressed rows bcomp[z] (bncomp[z] of them)
     uint32_t nb, q_ld, scores_ld, wlen;
+    uint32_t max_keys;     // the longest key list
     uint32_t wts_ld;       // k_attn_combine: floats per head of its dynamic LDS (>= every n_keys)
     uint32_t bpos[WH_POS_BATCH];
     uint32_t bncomp[WH_POS_BATCH];
@@ -267,10 +268,10 @@ struct wh_attn_pos {
     uint32_t n_win, n_comp, token_pos;
 };
 
-__device__ __forceinline__ wh_attn_pos wh_attn_resolve(const wh_attn_args& a) {
+__device__ __forceinline__ wh_attn_pos wh_attn_resolve(const wh_attn_args& a, uint32_t z) {
     wh_attn_pos v{a.q, a.win, a.comp, a.scores, a.out, a.n_win, a.n_comp, a.token_pos};
     if (a.nb) {
-        const uint32_t z = blockIdx.z, p = a.bpos[z], context = p + 1;
+        const uint32_t p = a.bpos[z], context = p + 1;
         const uint32_t ws = context > a.wlen ? context - a.wlen : 0u;
         v.q = a.q + (size_t)z * a.q_ld;
         v.out = a.out + (size_t)z * a.q_ld;
@@ -288,223 +289,360 @@ __device__ __forceinline__ const float* wh_attn_key(const wh_attn_args& a, const
     return j < v.n_win ? v.win + (size_t)j * a.win_ld : v.comp + (size_t)(j - v.n_win) * a.head_dim;
 }
 
-// The q rows of heads h0 .. h0 + 3 into LDS (zeros past the last head):
-// every thread's float4 loads are issued before the first store (a load
-// inside a loop or under a branch would be waited for one at a time).
-__device__ __forceinline__ void wh_attn_stage_q(const wh_attn_args& a, const wh_attn_pos& v, uint32_t h0, float* qs) {
-    constexpr int kPer = 4 * WH_ATTN_MAX_HEAD_DIM / 4 / 256;  // float4 per thread at most
-    const uint32_t hd = a.head_dim, n4 = hd;                   // 4 * hd floats = hd float4
-    float4 qv[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const uint32_t i4 = threadIdx.x + 256 * k, ic = i4 < n4 ? i4 : 0u, e = 4 * ic;
-        const uint32_t h = h0 + e / hd, hc = h < a.heads ? h : a.heads - 1;
-        qv[k] = *(const float4*)(v.q + (size_t)hc * hd + e % hd);
-    }
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const uint32_t i4 = threadIdx.x + 256 * k, e = 4 * i4;
-        if (i4 < n4) *(float4*)(qs + e) = h0 + e / hd < a.heads ? qv[k] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+// v(lane kI of each row of 16 lanes) * x: a DPP row broadcast is part of the
+// multiplication, so sixteen uniform factors in one register, the same in
+// every row, cost no instruction of their own.
+template <int kI>
+__device__ __forceinline__ float wh_mul_bcast(float v, float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + kI, 0xf, 0xf, true)) * x;
 }
 
 // scores[h][j] = (sum over d, in order, of q[h][d] * key_j[d]) * scale.
-// Grid (ceil(n_keys / 64), ceil(heads / 4)), 256 threads: wave w takes
-// head 4 * blockIdx.y + w, lane L key 64 * blockIdx.x + L.  Every thread
-// requests its share of the 64 keys (16 dims of each 64-dim chunk, up to 8
-// chunks) at once, so the launch waits for one memory round trip, not one
-// per chunk; the chunks then go through LDS 64 dims at a time (row stride
-// 65 floats: the lanes' reads of one dim fall in distinct banks), the four
-// heads' q rows once.
-#define WH_ATTN_PREFETCH 8u  // 64-dim chunks of a key requested together
+// Grid (ceil(n_keys / 64), ceil(heads / (4 kR)), positions), 256 threads: a
+// lane takes one key, a wave kR heads: two vector instructions per dim, head
+// and wave, which is what bounds a batch (q through scalar loads or readlane
+// was slower: 78 and 61 against 51 us for 64 heads x 628 keys of 32
+// positions, 80% of it vector issue; before, four heads a workgroup and both
+// factors of every product from LDS, 107 us).  The workgroup's 64 keys go through LDS 64 dims at a
+// time, two tiles in turn (one barrier a tile; row stride 68 floats: the
+// lanes' 16-byte reads fall in distinct banks), requested 8 (four heads
+// a wave: 4) tiles at a time so that the launch waits for one memory round
+// trip; the next dims' reads
+// are in flight while the current ones are added.  More heads per wave read
+// a key fewer times and leave fewer waves: see attn_launch.
+#define WH_ATTN_TILE_LD 68u  // floats per key of a score tile
+template <int kR>
 __global__ void __launch_bounds__(256) k_attn_scores(wh_attn_args a) {
-    __shared__ __align__(16) float qs[4 * WH_ATTN_MAX_HEAD_DIM];
-    __shared__ float tile[64 * 65];
-    const wh_attn_pos v = wh_attn_resolve(a);
+    constexpr int kPre = kR == 4 ? 4 : 8;  // tiles requested together
+    __shared__ __align__(16) float tile[2][64 * WH_ATTN_TILE_LD];
+    const wh_attn_pos v = wh_attn_resolve(a, blockIdx.z);
     const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const uint32_t h0 = blockIdx.y * 4, j0 = blockIdx.x * 64;
+    const uint32_t h0 = (blockIdx.y * 4 + wave) * kR, j0 = blockIdx.x * 64;
     const uint32_t nk = v.n_win + v.n_comp, hd = a.head_dim, n_ch = hd / 64;
     if (j0 >= nk) return;  // a batched launch's grid covers its longest key list
-    // staging: thread t copies 16 dims (t % 4) of key t / 4 of each chunk
-    const uint32_t kk = t >> 2, part = t & 3;
-    const bool kon = j0 + kk < nk;
-    const float* krow = kon ? wh_attn_key(a, v, j0 + kk) : nullptr;
-    float4 kv[WH_ATTN_PREFETCH][4];
+    // staging: thread t copies float4 t % 16 of keys t / 16 + 16 i of a tile
+    const uint32_t kk = t >> 4, f4 = t & 15;
+    const float* krow[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t j = j0 + kk + 16 * i;
+        krow[i] = wh_attn_key(a, v, j < nk ? j : j0) + 4 * f4;  // keys past the end: not stored
+    }
+    wh_f4 kv[kPre][4];
+    float qv[kPre][kR][4];  // of 16 dims each: lane i dim i % 16
     auto request = [&](uint32_t c0) {
 #pragma unroll
-        for (uint32_t c = 0; c < WH_ATTN_PREFETCH; ++c)
+        for (int c = 0; c < kPre; ++c) {
+            const uint32_t cc = c0 + c < n_ch ? c0 + c : 0u;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                kv[c][i] = kon && c0 + c < n_ch ? *(const float4*)(krow + 64 * (c0 + c) + part * 16 + 4 * i)
-                                                : make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int i = 0; i < 4; ++i) kv[c][i] = *(const wh_f4*)(krow[i] + 64 * cc);
+#pragma unroll
+            for (int r = 0; r < kR; ++r)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    qv[c][r][i] = v.q[(size_t)(h0 + r < a.heads ? h0 + r : a.heads - 1) * hd + 64 * cc + 16 * i +
+                                      (lane & 15)];
+        }
     };
     request(0);
-    wh_attn_stage_q(a, v, h0, qs);
-    const float* qrow = qs + wave * hd;
-    float s = 0.0f;
-    for (uint32_t c0 = 0; c0 < n_ch; c0 += WH_ATTN_PREFETCH) {
+    constexpr int kS = 16;  // dims per stage
+    float s[kR];
+#pragma unroll
+    for (int r = 0; r < kR; ++r) s[r] = 0.0f;
+    for (uint32_t c0 = 0; c0 < n_ch; c0 += kPre) {
         if (c0) request(c0);
-#pragma unroll
-        for (uint32_t c = 0; c < WH_ATTN_PREFETCH; ++c) {
+        wh_static_for<kPre>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
             if (c0 + c < n_ch) {  // uniform
-                __syncthreads();  // the previous chunk's reads are done (and q is staged)
+                float* dst = tile[c & 1];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float* d = tile + kk * 65 + part * 16 + 4 * i;
-                    d[0] = kv[c][i].x;
-                    d[1] = kv[c][i].y;
-                    d[2] = kv[c][i].z;
-                    d[3] = kv[c][i].w;
+                for (int i = 0; i < 4; ++i) *(wh_f4*)(dst + (kk + 16 * i) * WH_ATTN_TILE_LD + 4 * f4) = kv[c][i];
+                __syncthreads();  // and the reads of the tile before this one's last use are done
+                const float* src = tile[c & 1] + lane * WH_ATTN_TILE_LD;
+                wh_f4 kr[2][kS / 4];
+                auto read = [&](int b, int st) {
+#pragma unroll
+                    for (int i = 0; i < kS / 4; ++i) kr[b][i] = *(const wh_f4*)(src + kS * st + 4 * i);
+                };
+                read(0, 0);
+#pragma unroll
+                for (int st = 0; st < 64 / kS; ++st) {
+                    if (st + 1 < 64 / kS) read((st + 1) & 1, st + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    wh_static_for<kS>([&](auto ii) {
+                        constexpr int i = decltype(ii)::value;
+                        const float k = kr[st & 1][i >> 2][i & 3];
+#pragma unroll
+                        for (int r = 0; r < kR; ++r) s[r] = s[r] + wh_mul_bcast<i>(qv[c][r][st], k);
+                    });
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                __syncthreads();
-                const float* kr = tile + lane * 65;
-                const float* qc = qrow + 64 * (c0 + c);
-                for (uint32_t d = 0; d < 64; ++d) s = s + qc[d] * kr[d];
             }
+        });
+    }
+    const uint32_t j = j0 + lane;
+#pragma unroll
+    for (int r = 0; r < kR; ++r)
+        if (h0 + r < a.heads && j < nk) v.scores[(size_t)(h0 + r) * nk + j] = s[r] * a.scale;
+}
+
+// The keys' 64 dims d0 .. d0 + 63 of a workgroup through LDS, 64 keys a tile,
+// two tiles in turn, four requested ahead.
+struct wh_attn_tiles {
+    wh_f4 kv[4][4];
+    uint32_t kk, f4;  // thread t copies float4 t % 16 of keys t / 16 + 16 i
+    __device__ __forceinline__ void request(const wh_attn_args& a, const wh_attn_pos& v, uint32_t nk, uint32_t j0,
+                                            wh_f4 (&r)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t j = j0 + kk + 16 * i;  // past the last key: key 0's bytes, never used
+            r[i] = *(const wh_f4*)(wh_attn_key(a, v, j < nk ? j : 0u) + blockIdx.x * 64 + 4 * f4);
         }
     }
-    const uint32_t h = h0 + wave, j = j0 + lane;
-    if (h < a.heads && j < nk) v.scores[(size_t)h * nk + j] = s * a.scale;
+    // per tile, all threads: ahead(j0) for its keys' other loads, then
+    // body(tile, j0, keys).  Tiles come in fours and are requested whether
+    // they hold keys or not: with no load under a branch the compiler's waits
+    // cover exactly the tile that is stored (a load it cannot count makes
+    // every wait one for all loads, 1.3 us a tile).
+    template <class Ahead, class Body>
+    __device__ __forceinline__ void run(const wh_attn_args& a, const wh_attn_pos& v, uint32_t nk,
+                                        float (*tile)[64 * 64], Ahead ahead, Body body) {
+        for (uint32_t j0 = 0; j0 < nk; j0 += 256) {
+            wh_static_for<4>([&](auto ii) {
+                constexpr int i = decltype(ii)::value;
+                float* dst = tile[i & 1];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) *(wh_f4*)(dst + (kk + 16 * k) * 64 + 4 * f4) = kv[i][k];
+                ahead(ii, j0 + 64 * i);
+                request(a, v, nk, j0 + 64 * i + 256, kv[i]);
+                __syncthreads();  // and the reads of the tile before this one's last use are done
+                if (j0 + 64 * i < nk) body(ii, (const float*)tile[i & 1], j0 + 64 * i, min(64u, nk - (j0 + 64 * i)));
+            });
+        }
+    }
+    __device__ __forceinline__ void start(const wh_attn_args& a, const wh_attn_pos& v, uint32_t nk) {
+        kk = threadIdx.x >> 4;
+        f4 = threadIdx.x & 15;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) request(a, v, nk, 64 * i, kv[i]);
+    }
+};
+
+// f(sixteen b, key i, key's value) for keys 16 b + i < m of a tile, in order;
+// tp: the lane's dim of the tile's key 0.  A full tile is straight-line code
+// with the next sixteen keys' reads in flight.
+template <class F>
+__device__ __forceinline__ void wh_attn_keys(const float* tp, uint32_t m, F f) {
+    float x[2][16];
+    auto read = [&](int s, int b) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[s][i] = tp[64 * (16 * b + i)];
+    };
+    if (m == 64) {
+        read(0, 0);
+        wh_static_for<4>([&](auto bb) {
+            constexpr int b = decltype(bb)::value;
+            if constexpr (b < 3) read((b + 1) & 1, b + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            wh_static_for<16>([&](auto ii) { f(bb, ii, x[b & 1][decltype(ii)::value]); });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    } else {
+        wh_static_for<4>([&](auto bb) {
+            constexpr int b = decltype(bb)::value;
+            if (16 * b < m) {
+                read(0, b);  // past the last key: earlier bytes of the tile, not used
+                wh_static_for<16>([&](auto ii) {
+                    if (16 * b + decltype(ii)::value < m) f(bb, ii, x[0][decltype(ii)::value]);
+                });
+            }
+        });
+    }
+}
+
+// The inverse RoPE of dim d = 64 blockIdx.x + lane at token_pos
+// (E/compute.rs:4160-4197).
+struct wh_attn_rope {
+    float sn, cs;
+    bool any, on;  // the workgroup's dims (uniform) and this one are rope dims
+};
+__device__ __forceinline__ wh_attn_rope wh_attn_rope_of(const wh_attn_args& a, const wh_attn_pos& v, uint32_t d) {
+    wh_attn_rope r{0.0f, 1.0f, false, false};
+    const uint32_t first = blockIdx.x * 64, p = (d - a.nope_dim) / 2;
+    r.any = first + 63 >= a.nope_dim && first < a.nope_dim + 2 * a.pairs;
+    if (r.any) {
+        r.on = d >= a.nope_dim && p < a.pairs;
+        const float ang = (float)v.token_pos * (r.on ? a.inv_freqs[p] : 0.0f);
+        r.sn = -wh_sincosf_glibc(ang, 0);
+        r.cs = wh_sincosf_glibc(ang, 1);
+    }
+    return r;
+}
+
+// acc / den when den > 0, then the inverse RoPE; the lanes of a pair
+// exchange their values.
+__device__ __forceinline__ void wh_attn_finish(const wh_attn_args& a, const wh_attn_pos& v, const wh_attn_rope& rp,
+                                               float acc, float den, uint32_t h, uint32_t d) {
+    if (den > 0.0f) acc = acc / den;
+    if (rp.any) {
+        const float other = __shfl_xor(acc, 1, 64);
+        if (rp.on) acc = (d & 1) ? other * rp.sn + acc * rp.cs : acc * rp.cs - other * rp.sn;
+    }
+    if (h < a.heads) v.out[(size_t)h * a.head_dim + d] = acc;
 }
 
 // The rest of the window loop for 4 heads x 64 dims per workgroup (grid
-// (head_dim / 64, ceil(heads / 4)), 256 threads, 4 * wts_ld floats of
-// dynamic LDS; wave w = head, lane = dim):
+// (head_dim / 64, ceil(heads / 4), positions), 256 threads, 4 * wts_ld floats
+// of dynamic LDS; wave w = head, lane = dim):
 //   max = the largest score (NaN scores never win, E/compute.rs:4125-4127);
 //   w_j = expf(score_j - max); denom = expf(sink - max) (if a sink) +
 //   (sequential sum of w_j); out_d = sequential sum of w_j * key_j[d] from 0;
-//   out_d /= denom when denom > 0; then the inverse RoPE of the output's
-//   rope dims at token_pos (E/compute.rs:4160-4197).
-// The keys' 64 dims of the workgroup go through LDS 128 keys at a time,
-// staged once for the four heads; the first 128 are requested before the
-// softmax pass.
-#define WH_ATTN_KCHUNK 128u
+//   out_d /= denom when denom > 0; then the inverse RoPE.
+// For few positions: each of the head_dim / 64 workgroups of a head makes its
+// weights again and, beside its chain of weighted keys, the denominator's,
+// which costs less than a launch: four instructions a key.
 __global__ void __launch_bounds__(256) k_attn_combine(wh_attn_args a) {
-    extern __shared__ __align__(16) float wts[];  // [4][wts_ld], wts_ld a multiple of 4
-    __shared__ __align__(16) float tile[WH_ATTN_KCHUNK * 64];
-    __shared__ float res[4 * 64];
-    __shared__ float denom_s[4];
-    const wh_attn_pos v = wh_attn_resolve(a);
+    extern __shared__ __align__(16) float wts[];  // [4][wts_ld]
+    __shared__ __align__(16) float tile[2][64 * 64];
+    const wh_attn_pos v = wh_attn_resolve(a, blockIdx.z);
     const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const uint32_t h = blockIdx.y * 4 + wave, d = blockIdx.x * 64 + lane;
     const uint32_t nk = v.n_win + v.n_comp;
     const bool hon = h < a.heads;
-    // staging: thread t copies dims 32 (t % 2) .. + 31 of key t / 2 of the chunk
-    const uint32_t kk = t >> 1, half = t & 1;
-    float4 kr[8];
-    auto request = [&](uint32_t c0) {
-        const bool on = c0 + kk < nk;
-        const float* src = on ? wh_attn_key(a, v, c0 + kk) + blockIdx.x * 64 + 32 * half : nullptr;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) kr[i] = on ? *(const float4*)(src + 4 * i) : make_float4(0.f, 0.f, 0.f, 0.f);
-    };
-    request(0);
+    const uint32_t hc = hon ? h : a.heads - 1;
+    const float sink = a.sink ? a.sink[hc] : 0.0f;
     float* w = wts + wave * a.wts_ld;
-    const float* sc = v.scores + (size_t)(hon ? h : 0) * nk;
+    const float* sc = v.scores + (size_t)hc * nk;
     float mx = -__uint_as_float(0x7f800000u);
-    uint32_t j = lane;
-    // four scores' loads at a time (sc is a valid row for every wave)
-    for (; j + 192 < nk; j += 256) {
+    // four scores' loads at a time
+    for (uint32_t j = lane; j < nk; j += 256) {
         float sv[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) sv[k] = sc[j + 64 * k];
+        for (int k = 0; k < 4; ++k) sv[k] = sc[j + 64 * k < nk ? j + 64 * k : j];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const float x = hon ? sv[k] : 0.0f;
-            w[j + 64 * k] = x;
-            mx = fmaxf(mx, x);
+            if (j + 64 * k < nk) w[j + 64 * k] = sv[k];
+            mx = fmaxf(mx, sv[k]);
         }
     }
-    if (j + 64 < nk) {
-        const float s0 = sc[j], s1 = sc[j + 64];
-        const float x0 = hon ? s0 : 0.0f, x1 = hon ? s1 : 0.0f;
-        w[j] = x0;
-        w[j + 64] = x1;
-        mx = fmaxf(fmaxf(mx, x0), x1);
-        j += 128;
-    }
-    for (; j < nk; j += 64) {
-        const float x = hon ? sc[j] : 0.0f;
-        w[j] = x;
-        mx = fmaxf(mx, x);
-    }
+    wh_attn_tiles tiles;
+    tiles.start(a, v, nk);
     mx = wh_wave_max(mx);
     for (uint32_t j = lane; j < nk; j += 64) w[j] = wh_expf_glibc(w[j] - mx, kExpTab, kExpfExc, WH_EXPF_EXC_COUNT);
-    __syncthreads();
-    if (lane == 0) {
-        const float ws = wh_ordered_sum_lds(w, nk, 0.0f);
-        float den = 0.0f;
-        if (a.sink && hon) den = den + wh_expf_glibc(a.sink[h] - mx, kExpTab, kExpfExc, WH_EXPF_EXC_COUNT);
-        denom_s[wave] = den + ws;
-    }
-    float acc = 0.0f;
-    for (uint32_t c0 = 0; c0 < nk; c0 += WH_ATTN_KCHUNK) {
-        if (c0) {
-            __syncthreads();  // the previous chunk's reads are done
-            request(c0);
-        }
-        float* dst = tile + kk * 64 + 32 * half;
+    const float den0 = a.sink ? 0.0f + wh_expf_glibc(sink - mx, kExpTab, kExpfExc, WH_EXPF_EXC_COUNT) : 0.0f;
+    float acc = 0.0f, ws = 0.0f;
+    tiles.run(a, v, nk, tile, [](auto, uint32_t) {}, [&](auto, const float* tl, uint32_t j0, uint32_t m) {
+        float wv[4];  // of 16 keys each
 #pragma unroll
-        for (int i = 0; i < 8; ++i) *(float4*)(dst + 4 * i) = kr[i];
+        for (int i = 0; i < 4; ++i) wv[i] = w[min(j0 + 16 * i + (lane & 15), nk - 1)];
+        const float* tp = tl + lane;
+        wh_attn_keys(tp, m, [&](auto bb, auto ii, float x) {
+            constexpr int b = decltype(bb)::value, i = decltype(ii)::value;
+            ws = ws + wh_mul_bcast<i>(wv[b], 1.0f);
+            acc = acc + wh_mul_bcast<i>(wv[b], x);
+        });
+    });
+    wh_attn_finish(a, v, wh_attn_rope_of(a, v, d), acc, den0 + ws, h, d);
+}
+
+// The same as two launches, for many positions: the weights once per head ...
+// Grid (heads, positions), 256 threads.  The weights replace the scores; the
+// denominator waits in the first dim of each 64-dim block of the output,
+// which k_attn_weighted's wave of that block reads before it writes.
+__global__ void __launch_bounds__(256) k_attn_softmax(wh_attn_args a) {
+    constexpr int kPer = WH_ATTN_MAX_KEYS / 256;
+    __shared__ __align__(16) wh_osum_lds<WH_ATTN_MAX_KEYS / 32, 32> os;
+    __shared__ float red[4];
+    const uint32_t t = threadIdx.x, h = blockIdx.x;
+    const wh_attn_pos v = wh_attn_resolve(a, blockIdx.y);
+    const uint32_t nk = v.n_win + v.n_comp;
+    float* sc = v.scores + (size_t)h * nk;
+    float x[kPer];
+    float mx = -__uint_as_float(0x7f800000u);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) x[k] = 256 * k < nk ? sc[min(t + 256 * k, nk - 1)] : mx;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) mx = fmaxf(mx, x[k]);
+    mx = wh_wave_max(mx);
+    if ((t & 63) == 0) red[t >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        if (256 * k < nk) {  // uniform
+            x[k] = wh_expf_glibc(x[k] - mx, kExpTab, kExpfExc, WH_EXPF_EXC_COUNT);
+            if (t + 256 * k < nk) sc[t + 256 * k] = x[k];
+        }
+    }
+    // the weights' sequential sum: one lane up to 512 (as in k_rowpost)
+    auto sum = [&](auto l) {
+        constexpr int kL = decltype(l)::value;
+        auto& s = *(wh_osum_lds<kL, 32>*)&os;
+#pragma unroll
+        for (int k = 0; k < 32 * kL / 256; ++k) s.rows[wh_osum_at<kL>(t + 256 * k)] = t + 256 * k < nk ? x[k] : -0.0f;
+        return wh_ordered_sum_wg<256, kL, 32>(s, 0.0f);
+    };
+    float ws = 0.0f;
+    if (nk <= 512) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (t + 256 * k < nk) os.rows[t + 256 * k] = x[k];
         __syncthreads();
-        const uint32_t m = min(WH_ATTN_KCHUNK, nk - c0);
-        if (hon) {
-            // blocks of 16 keys: the weights (broadcast) and the lane's 16
-            // key values of the next block are read while the current block
-            // is added; a full chunk is straight-line code, in which the
-            // compiler counts the reads in flight exactly
-            const float* wc = w + c0;
-            float4 wa[2][4];
-            float ta[2][16];
-            auto rdb = [&](int sl, uint32_t jb) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) wa[sl][i] = *(const float4*)(wc + 16 * jb + 4 * i);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) ta[sl][i] = tile[(16 * jb + i) * 64 + lane];
-            };
-            auto addb = [&](int sl) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    acc = acc + wa[sl][i].x * ta[sl][4 * i];
-                    acc = acc + wa[sl][i].y * ta[sl][4 * i + 1];
-                    acc = acc + wa[sl][i].z * ta[sl][4 * i + 2];
-                    acc = acc + wa[sl][i].w * ta[sl][4 * i + 3];
-                }
-            };
-            const uint32_t mb = m / 16;
-            if (mb == WH_ATTN_KCHUNK / 16) {
-                rdb(0, 0);
-#pragma unroll
-                for (int b = 0; b < (int)(WH_ATTN_KCHUNK / 16); ++b) {
-                    if (b + 1 < (int)(WH_ATTN_KCHUNK / 16)) rdb((b + 1) & 1, b + 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                    addb(b & 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            } else {
-                for (uint32_t b = 0; b < mb; ++b) {
-                    rdb(0, b);
-                    addb(0);
-                }
-            }
-            for (uint32_t j = 16 * mb; j < m; ++j) acc = acc + wc[j] * tile[j * 64 + lane];
-        }
+        if (t == 0) ws = wh_ordered_sum_lds(os.rows, nk, 0.0f);
+    } else if (nk <= 1024) {
+        ws = sum(std::integral_constant<int, 32>());
+    } else {
+        ws = sum(std::integral_constant<int, WH_ATTN_MAX_KEYS / 32>());
     }
-    __syncthreads();
-    const float den = denom_s[wave];
-    if (den > 0.0f) acc = acc / den;
-    res[wave * 64 + lane] = acc;
-    __syncthreads();
-    // inverse RoPE: the even lane of a pair in [nope_dim, head_dim) rotates it
-    if (d >= a.nope_dim && ((d - a.nope_dim) & 1) == 0 && (d - a.nope_dim) / 2 < a.pairs) {
-        const uint32_t p = (d - a.nope_dim) / 2;
-        const float ang = (float)v.token_pos * a.inv_freqs[p];
-        const float sn = -wh_sincosf_glibc(ang, 0);
-        const float cs = wh_sincosf_glibc(ang, 1);
-        const float e = res[wave * 64 + lane], o = res[wave * 64 + lane + 1];
-        res[wave * 64 + lane] = e * cs - o * sn;
-        res[wave * 64 + lane + 1] = e * sn + o * cs;
+    if (t == 0) {
+        const float den0 =
+            a.sink ? 0.0f + wh_expf_glibc(a.sink[h] - mx, kExpTab, kExpfExc, WH_EXPF_EXC_COUNT) : 0.0f;
+        for (uint32_t b = 0; b < a.head_dim; b += 64) v.out[(size_t)h * a.head_dim + b] = den0 + ws;
     }
-    __syncthreads();
-    if (hon) v.out[(size_t)h * a.head_dim + d] = res[wave * 64 + lane];
+}
+
+// ... and the weighted sums: grid (head_dim / 64, ceil(heads / (4 kR)),
+// positions), a wave kR heads x 64 dims: two vector instructions per key and
+// head, 83% of the launch (64 heads x 628 keys of 32 positions: 63 us and 12 us
+// for the weights, 201 us when every 4 heads x 64 dims did both); the wave's
+// heads share the key's way through LDS.
+template <int kR>
+__global__ void __launch_bounds__(256) k_attn_weighted(wh_attn_args a) {
+    __shared__ __align__(16) float tile[2][64 * 64];
+    const wh_attn_pos v = wh_attn_resolve(a, blockIdx.z);
+    const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const uint32_t h0 = (blockIdx.y * 4 + wave) * kR, d = blockIdx.x * 64 + lane;
+    const uint32_t nk = v.n_win + v.n_comp;
+    wh_attn_tiles tiles;
+    tiles.start(a, v, nk);
+    const float* w[kR];
+    float den[kR], acc[kR];
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+        const uint32_t h = h0 + r < a.heads ? h0 + r : a.heads - 1;
+        w[r] = v.scores + (size_t)h * nk;
+        den[r] = h0 + r < a.heads ? v.out[(size_t)h * a.head_dim + blockIdx.x * 64] : 0.0f;
+        acc[r] = 0.0f;
+    }
+    float wn[2][kR][4];  // the weights of this tile and the next, 16 keys each
+    auto weights = [&](float (&d)[kR][4], uint32_t j0) {
+#pragma unroll
+        for (int r = 0; r < kR; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[r][i] = w[r][min(j0 + 16 * i + (lane & 15), nk - 1)];
+    };
+    weights(wn[0], 0);
+    tiles.run(
+        a, v, nk, tile, [&](auto t0, uint32_t j0) { weights(wn[(decltype(t0)::value + 1) & 1], j0 + 64); },
+        [&](auto t0, const float* tl, uint32_t j0, uint32_t m) {
+            wh_attn_keys(tl + lane, m, [&](auto bb, auto ii, float x) {
+                constexpr int b = decltype(bb)::value, i = decltype(ii)::value;
+#pragma unroll
+                for (int r = 0; r < kR; ++r)
+                    acc[r] = acc[r] + wh_mul_bcast<i>(wn[decltype(t0)::value & 1][r][b], x);
+            });
+        });
+    const wh_attn_rope rp = wh_attn_rope_of(a, v, d);
+#pragma unroll
+    for (int r = 0; r < kR; ++r) wh_attn_finish(a, v, rp, acc[r], den[r], h0 + r, d);
 }

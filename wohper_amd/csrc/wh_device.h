@@ -11,9 +11,24 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "libm_emul.h"
 
 typedef float wh_f2 __attribute__((ext_vector_type(2)));
+typedef float wh_f4 __attribute__((ext_vector_type(4)));
+
+// f(integral_constant 0), ..., f(integral_constant kN - 1): a loop whose
+// register arrays are indexed by constants whatever the unroller makes of it.
+template <class F, int... kI>
+__device__ __forceinline__ void wh_static_for_seq(F&& f, std::integer_sequence<int, kI...>) {
+    (f(std::integral_constant<int, kI>()), ...);
+}
+template <int kN, class F>
+__device__ __forceinline__ void wh_static_for(F&& f) {
+    wh_static_for_seq(f, std::make_integer_sequence<int, kN>());
+}
 
 // ---------------------------------------------------------------- FP8 codes
 // gfx950 converts OCP E4M3 (bias 7) in hardware.  Codes 0x7F/0xFF are NaN
