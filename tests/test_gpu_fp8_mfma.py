@@ -226,3 +226,83 @@ def test_pair_equals_two_multi_calls(ctx, oracle, exact):
             check(oracle, w, rows, cols, s, xs, g)
     for t in ts:
         ctx.release(t)
+
+
+@pytest.mark.parametrize("rows,cols,n,r0,r1,special", [
+    (2304, 8192, 33, 0, 2304, False),     # 32-input blocks, the second with one input
+    (2560, 8192, 40, 16, 2544, True),     # a row range off the 64- and 256-row grids, all codes
+    (4096, 2048, 144, 0, 4096, False),    # 48-input blocks
+    (4096, 4096, 250, 0, 4080, False),    # 64-input blocks, the last partial
+])
+def test_fp8_mfma_wide_against_oracle(ctx, oracle, rows, cols, n, r0, r1, special):
+    """k_fp8_mm_wide at the edges of its row and input blocks, within the
+    bound of any fp32 summation order."""
+    case = wl.fp8_gemv_case(rows, cols, seed=rows + n)
+    w = case.w.copy()
+    if special:
+        w[::5, ::7], w[2::5, 3::7] = 0x7F, 0xFF
+    t = ctx.store_fp8(w, rows, cols, case.scales, rows // 128, cols // 128, wohper_amd.SCALE_F32)
+    xs = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    ys = run_multi(ctx, t, xs, r0, r1, cols)
+    wd = dense(oracle, w, case.scales)
+    for i in {0, 1, 15, 16, 31, 32, n // 2, n - 2, n - 1}:
+        check(oracle, w, rows, cols, case.scales, xs[i:i + 1], ys[i:i + 1], r0, r1, wd)
+    ctx.release(t)
+
+
+@pytest.mark.parametrize("ue8m0", [False, True])
+def test_fp8_mfma_wide_one_hot_exact(ctx, oracle, ue8m0):
+    """One one-hot input per column, in one call: every weight and scale comes
+    out exactly at its own row, column and input."""
+    rows, cols = 1280, 1024
+    rng = np.random.default_rng(5)
+    w = rng.integers(0, 256, (rows, cols)).astype(np.uint8)
+    e = rng.integers(-6, 3, (rows // 128, cols // 128))
+    s = np.exp2(e).astype(np.float32)
+    fmt = wohper_amd.SCALE_UE8M0 if ue8m0 else wohper_amd.SCALE_F32
+    t = ctx.store_fp8(w, rows, cols, (e + 127).astype(np.uint8) if ue8m0 else s, rows // 128, cols // 128, fmt)
+    ys = run_multi(ctx, t, np.eye(cols, dtype=np.float32), 0, rows, cols)
+    fp8, _, _, _ = oracle.luts()
+    want = (fp8[w] * s.repeat(128, 0).repeat(128, 1)).T.astype(np.float32)
+    assert np.array_equal(ys, want), int(np.count_nonzero(ys != want))
+    ctx.release(t)
+
+
+@pytest.mark.parametrize("n", [49, 128, 193])
+def test_fp8_mfma_wide_pair_and_groups(ctx, n):
+    """wq_a + wkv in one launch with two k splits, and wo_a's row groups, are
+    the single calls bit for bit."""
+    cols = 4096
+    rng = np.random.default_rng(n)
+    cases = [wl.fp8_gemv_case(r, cols, seed=r + n) for r in (1024, 512, 8192)]
+    ts = [ctx.store_fp8(k.w, k.w.shape[0], cols, k.scales, k.w.shape[0] // 128, cols // 128, wohper_amd.SCALE_F32)
+          for k in cases]
+    x = rng.standard_normal((n, 8 * cols)).astype(np.float32)
+    xd, yd = ctx.device_alloc(x.nbytes), ctx.device_alloc(4 * n * 8192)
+    ctx.to_device(xd, x)
+    rows = (1024, 512)
+    y1 = yd + 4 * n * rows[0]
+
+    def fetch(p, r):
+        out = np.empty((n, r), np.float32)
+        ctx.from_device(out, p)
+        return out
+    for t, r, y in zip(ts, rows, (yd, y1)):
+        ctx.fp8_gemv_multi_async(t, 0, r, xd, n, 8 * cols, y, r)
+    want = [fetch(yd, rows[0]), fetch(y1, rows[1])]
+    for _ in range(2):  # the arrival counters are back at zero
+        ctx.fp8_gemv_multi_pair_async(ts[0], 0, rows[0], yd, rows[0], ts[1], 0, rows[1], y1, rows[1], xd, n, 8 * cols)
+        assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32))
+                   for a, b in zip(want, (fetch(yd, rows[0]), fetch(y1, rows[1]))))
+    ctx.fp8_gemv_multi_groups_async(ts[2], 0, 8192, 1024, xd, cols, n, 8 * cols, yd, 8192)
+    got = fetch(yd, 8192)
+    wd = np.empty((n, 1024), np.float32)
+    for g in (0, 7):
+        ctx.fp8_gemv_multi_async(ts[2], g * 1024, (g + 1) * 1024, xd + 4 * g * cols, n, 8 * cols, yd, 1024)
+        ctx.from_device(wd, yd)
+        # another k split: the sums' order only
+        assert np.allclose(got[:, g * 1024:(g + 1) * 1024], wd, rtol=1e-4, atol=1e-5 * np.abs(wd).max())
+    for t in ts:
+        ctx.release(t)
+    ctx.device_free(xd)
+    ctx.device_free(yd)

@@ -71,6 +71,9 @@ struct wh_fp8mm_args {
     const void* scales2;
     float* y2;
     uint32_t row_start2, row_end2, y2_stride, rb_first;
+    // k_fp8_mm_wide only: the second tensor's k split, which may be another,
+    // and the splits between two blocks' partial tiles (the larger count)
+    uint32_t kc2, splits2, ws_splits;
 };
 
 // Two f32 to two bf16, each rounded to nearest even (v_cvt_pk_bf16_f32).
@@ -287,4 +290,199 @@ __global__ void __launch_bounds__(512, WH_FP8MM_WG_PER_CU) k_fp8_mm(wh_fp8mm_arg
             if (!(fabsf(sum[k]) <= 3.4028235e38f)) atomicOr(a.status, WH_ST_NONFINITE_OUTPUT);
         }
     }
+}
+
+// More than 16 inputs (k_fp8_mm would read and decode every weight byte once
+// per 16 of them, and feed each MFMA a fragment of its own from LDS: 1 KB in
+// 16 cycles from each of four SIMDs, twice what LDS delivers).  Here a wave
+// holds 64 rows x 16 kT inputs: a fragment of inputs feeds four MFMAs, a decoded
+// weight 3 kT of them.  The products, their order and the k split are
+// k_fp8_mm's, so the results are the same bits.
+//
+// Bound by the MFMAs (three a product) and the input split of the same waves:
+// 192 inputs of 32768 x 1024, 8192 x 4096 in 8 groups and 4096 x 8192 take 45,
+// 48 and 47 us (850, 806 and 823 TFLOP/s of bf16 products; a large library
+// product reaches 1200 here), against 86, 116 and 92 us in k_fp8_mm.
+//
+// Workgroup: 4 waves x 64 rows, two a CU, so that one stages while the other
+// multiplies.  A stage is 128 columns (256 for 32 inputs) of the inputs' three
+// planes, 48 KB at most; the next stage's inputs and the next group's weights
+// load while a stage is multiplied.  A lane of input tile `col` keeps the
+// staging stores of 16 lanes contiguous.
+#define WH_FP8MMW_ROWS 256u  // rows per workgroup: 4 waves x 64
+
+// grid (row blocks, most splits of a tensor, blocks of 16 kT inputs), 256 threads
+template <bool kSpecial, bool kScaleU8, int kT>
+__global__ void __launch_bounds__(256, 2) k_fp8_mm_wide(wh_fp8mm_args a) {
+    static_assert(kT >= 2 && kT <= 4, "a stage is at most 64 inputs x groups");
+    constexpr uint32_t kGS = kT == 2 ? 2 : 1;  // 128-column groups per LDS stage
+    constexpr int kR = 4;                      // row tiles of 16 per wave
+    constexpr uint32_t kRows = WH_FP8MMW_ROWS;
+    constexpr uint32_t kTok = 16 * kT;    // inputs per workgroup
+    constexpr uint32_t P = 16 * kGS * kTok * 8;  // bf16 of one plane
+    __shared__ __align__(16) uint16_t xs[3 * P];  // [hi | mid | lo][group][m][q][input][8]
+    const uint32_t rb = blockIdx.x, ks = blockIdx.y, tb = blockIdx.z;
+    const uint32_t wave = threadIdx.x >> 6, L = threadIdx.x & 63, q = L >> 4, col = L & 15;
+    const bool t2 = rb >= a.rb_first;
+    const uint32_t splits = t2 ? a.splits2 : a.splits;
+    if (ks >= splits) return;
+    const uint8_t* const W = t2 ? a.w2 : a.w;
+    const void* const SC = t2 ? a.scales2 : a.scales;
+    float* const Y = t2 ? a.y2 : a.y;
+    const uint32_t row_start = t2 ? a.row_start2 : a.row_start, row_end = t2 ? a.row_end2 : a.row_end;
+    const uint32_t y_stride = t2 ? a.y2_stride : a.y_stride;
+    const uint32_t rbl = t2 ? rb - a.rb_first : rb;
+    const uint32_t r0 = row_start + rbl * kRows + 16 * kR * wave;  // the wave's first row
+    const uint32_t grp = a.xg_shift < 31 ? (rbl * kRows) >> a.xg_shift : 0;
+    const uint32_t G = (t2 ? a.kc2 : a.kc) >> 7, g0 = ks * G;
+    // staging: thread (group, input tile | h, half | input of the tile); inputs
+    // past the end stage the last one's values, whose sums are not stored
+    const uint32_t sgs = kT == 2 ? wave >> 1 : 0, stt = kT == 2 ? wave & 1 : wave;
+    const uint32_t sh = q >> 1, shalf = q & 1;
+    const uint32_t stok = tb * kTok + 16 * stt + col;
+    const bool stager = kT != 3 || wave < 3;
+    const float* const xr = a.x + (size_t)(stok < a.n ? stok : a.n - 1) * a.x_stride + (size_t)grp * a.xg_stride +
+                            (size_t)(g0 + sgs) * 128 + 8 * sh + 4 * shalf;
+    float4 xv[8];
+    auto load_x = [&](uint32_t stage) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) xv[c] = *(const float4*)(xr + (size_t)stage * (128 * kGS) + 16 * c);
+    };
+    // row tile i: rows r0 + 16 i .. (rows past the end load row_start's bytes; not stored)
+    const uint8_t* wrow[kR];
+#pragma unroll
+    for (int i = 0; i < kR; ++i) {
+        const uint32_t row = r0 + 16 * i + col;
+        wrow[i] = W + (size_t)(row < row_end ? row : row_start) * a.cols + (size_t)g0 * 128 + 32 * q;
+    }
+    // lane i < kR loads tile i's scale of each group
+    const uint32_t trow = r0 + 16 * (L & (kR - 1)) < row_end ? r0 + 16 * (L & (kR - 1)) : row_end - 1;
+    const size_t srow = (size_t)(trow >> a.row_group_shift) * a.scale_cols + g0;
+    if (stager) load_x(0);
+    float sv = wh_fp8mm_scale<kScaleU8>(SC, srow);
+    uint4 w[kR][2];
+#pragma unroll
+    for (int i = 0; i < kR; ++i) {
+        w[i][0] = *(const uint4*)(wrow[i]);
+        w[i][1] = *(const uint4*)(wrow[i] + 16);
+    }
+    wh_f32x4 total[kR][kT];
+#pragma unroll
+    for (int i = 0; i < kR; ++i)
+#pragma unroll
+        for (int t = 0; t < kT; ++t) total[i][t] = (wh_f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t n_stages = G / kGS;
+    for (uint32_t s = 0; s < n_stages; ++s) {
+        if (s) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (!stager) break;
+            const float v[8] = {((const float*)&xv[0])[i], ((const float*)&xv[1])[i], ((const float*)&xv[2])[i],
+                                ((const float*)&xv[3])[i], ((const float*)&xv[4])[i], ((const float*)&xv[5])[i],
+                                ((const float*)&xv[6])[i], ((const float*)&xv[7])[i]};
+            uint4 hi, mid, lo;
+            wh_split3_x8(v, hi, mid, lo);
+            const uint32_t l = 4 * shalf + i, m = (2 * l + sh) & 3, lq = l >> 1;
+            const uint32_t off = (((sgs * 4 + m) * 4 + lq) * kTok + 16 * stt + col) * 8;
+            *(uint4*)(xs + off) = hi;
+            *(uint4*)(xs + P + off) = mid;
+            *(uint4*)(xs + 2 * P + off) = lo;
+        }
+        __syncthreads();
+        if (stager && s + 1 < n_stages) load_x(s + 1);
+#pragma unroll
+        for (uint32_t gs = 0; gs < kGS; ++gs) {
+            const uint32_t gi = s * kGS + gs;
+            const uint32_t gn = gi + 1 < G ? gi + 1 : gi;  // the group loaded meanwhile
+            const float sc = sv;
+            sv = wh_fp8mm_scale<kScaleU8>(SC, srow + gn);
+            wh_f32x4 acc[kR][kT];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                wh_bf16x8 av[kR];
+#pragma unroll
+                for (int i = 0; i < kR; ++i) {
+                    const uint4 d = w[i][m >> 1];
+                    av[i] = wh_fp8_bf16x8<kSpecial>(m & 1 ? d.z : d.x, m & 1 ? d.w : d.y);
+                }
+                if (m & 1) {
+#pragma unroll
+                    for (int i = 0; i < kR; ++i)
+                        w[i][m >> 1] = *(const uint4*)(wrow[i] + (size_t)gn * 128 + 16 * (m >> 1));
+                }
+#pragma unroll
+                for (int t = 0; t < kT; ++t)
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) {
+                        const wh_bf16x8 b =
+                            *(const wh_bf16x8*)(xs + p * P + (((gs * 4 + m) * 4 + q) * kTok + 16 * t + col) * 8);
+#pragma unroll
+                        for (int i = 0; i < kR; ++i)
+                            acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                b, av[i], m == 0 && p == 0 ? (wh_f32x4){0.0f, 0.0f, 0.0f, 0.0f} : acc[i][t], 0, 0, 0);
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < kR; ++i) {
+                const float f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), i));
+#pragma unroll
+                for (int t = 0; t < kT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) total[i][t][r] = __builtin_fmaf(acc[i][t][r], f, total[i][t][r]);
+            }
+        }
+    }
+    // D[4 q + r][col]: input 4 q + r of the tile, row `col` of the tile
+    if (splits > 1) {
+        // partial tiles in register order; the last workgroup of the block sums
+        // the splits in order
+        constexpr uint32_t kTile = kRows * kTok;
+        const size_t tile = ((size_t)tb * a.row_blocks + rb) * a.ws_splits;
+        float* const wsp = a.ws + (tile + ks) * kTile + (size_t)wave * (kTile / 4) + L;
+#pragma unroll
+        for (int i = 0; i < kR; ++i)
+#pragma unroll
+            for (int t = 0; t < kT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) wh_store_coherent(wsp + ((i * kT + t) * 4 + r) * 64, total[i][t][r]);
+        wh_stores_done();
+        __syncthreads();
+        uint32_t* const last = (uint32_t*)xs;
+        if (threadIdx.x == 0) {
+            uint32_t* cnt = a.cnt + (size_t)tb * a.row_blocks + rb;
+            *last = wh_arrive(cnt) + 1 == splits;
+            if (*last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (!*last) return;
+        const float* const wt = a.ws + tile * kTile + (size_t)wave * (kTile / 4) + L;
+        for (uint32_t sp = 0; sp < splits; ++sp) {
+#pragma unroll
+            for (int i = 0; i < kR; ++i)
+#pragma unroll
+                for (int t = 0; t < kT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float v = wh_load_coherent(wt + (size_t)sp * kTile + ((i * kT + t) * 4 + r) * 64);
+                        total[i][t][r] = sp == 0 ? v : total[i][t][r] + v;
+                    }
+        }
+    }
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kR; ++i) {
+        const uint32_t row = r0 + 16 * i + col;
+        if (row >= row_end) continue;
+#pragma unroll
+        for (int t = 0; t < kT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t tok = tb * kTok + 16 * t + 4 * q + r;
+                if (tok < a.n) {
+                    Y[(size_t)tok * y_stride + (row - row_start)] = total[i][t][r];
+                    bad |= !(fabsf(total[i][t][r]) <= 3.4028235e38f);
+                }
+            }
+    }
+    if (bad) atomicOr(a.status, WH_ST_NONFINITE_OUTPUT);
 }
