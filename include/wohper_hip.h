@@ -650,7 +650,9 @@ int wh_act_quant_dequant_async(wh_ctx* ctx, float* values_dev, size_t n, size_t 
  * logit sink_dev[h] in the denominator, out = sum of weight * key in key
  * order, divided by the denominator when positive, then the inverse RoPE of
  * the rope dims [nope_dim, nope_dim + 2 pairs) at token_pos.  scores_dev:
- * heads * (n_window + n_comp) floats of scratch.  head_dim a multiple of 64,
+ * heads * (n_window + n_comp) floats of scratch.  With exact numerics off
+ * (wh_set_exact_numerics(ctx, 0)), q_dev 16-byte aligned and at most 256
+ * heads, the same sums run on f32 matrix instructions in another order.  head_dim a multiple of 64,
  * at most 1024; at most 2048 keys; window_dev and comp_dev 16-byte aligned
  * and window_stride a multiple of 4 (WH_INVALID_ARGUMENT otherwise). */
 int wh_window_attention_async(wh_ctx* ctx, const float* q_dev, size_t heads, size_t head_dim, size_t nope_dim,
@@ -751,7 +753,7 @@ int wh_hc_post_async(wh_ctx* ctx, const float* y_dev, const float* residual_dev,
  *     hidden = hc_post(z, hidden').
  * Every step is the kernel of its own entry point, so the layer is
  * bit-identical to the reference under exact numerics; with exact numerics
- * off the FP8 projections, the expert matvecs and hc_pre's sums take the
+ * off the FP8 projections, the attention's sums, the expert matvecs and hc_pre's sums take the
  * order-free kernels (the router keeps the reference order).  Nothing is
  * read back to the host: the whole layer can be captured (wh_graph_begin).
  * hidden_dev 16-byte aligned; the norm weights are bf16 (NULL: plain RMS

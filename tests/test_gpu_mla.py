@@ -179,6 +179,78 @@ def test_window_attention_shapes_bit_exact(ctx, oracle, dev, heads, hd, nope, pa
     assert np.array_equal(bits(dev.get(outp, (heads, hd))), bits(want))
 
 
+def _order_free_attention(ctx, dev, q, win, comp, sk, inv, nope, pairs, pos):
+    heads, hd = q.shape
+    nk = len(win) + len(comp)
+    outp, scp = dev.empty(heads * hd * 4), dev.empty(heads * nk * 4)
+    args = (dev.put(q), heads, hd, nope, dev.put(win) if len(win) else 0, len(win), hd,
+            dev.put(comp) if len(comp) else 0, len(comp), dev.put(sk), dev.put(inv), pairs, pos, scp, outp)
+    outs = {}
+    for exact in (True, False):
+        ctx.set_exact_numerics(exact)
+        try:
+            ctx.window_attention_async(*args)
+            ctx.synchronize()
+        finally:
+            ctx.set_exact_numerics(True)
+        outs[exact] = dev.get(outp, (heads, hd))
+    return outs
+
+
+@pytest.mark.parametrize("heads,hd,nope,pairs", [(1, 64, 0, 32), (3, 128, 70, 20), (16, 192, 128, 32),
+                                                 (65, 1024, 960, 32), (128, 512, 512, 0)])
+@pytest.mark.parametrize("n_win,n_comp", [(0, 1), (15, 0), (16, 1), (32, 0), (63, 2), (128, 385), (128, 1920)])
+def test_window_attention_order_free(ctx, dev, heads, hd, nope, pairs, n_win, n_comp):
+    """The matrix-instruction kernels at the edges of their head, key and dim
+    tiles, against 64 bits.  Bound, with u = 2^-24: a score of hd terms in any
+    order is within d = (hd + 2) u sum|q k| scale of its value, a weight within
+    2 d + 8 u of its own relative to the denominator's, and the sums over keys
+    add 2 (n + 2) u; the rotation mixes a pair."""
+    rng = np.random.default_rng(heads * 7 + n_comp)
+    inv = (10000.0 ** -(np.arange(max(pairs, 1)) / max(pairs, 1))).astype(np.float32)
+    q = (rng.standard_normal((heads, hd)) * 3).astype(np.float32)
+    win = rng.standard_normal((n_win, hd)).astype(np.float32)
+    comp = rng.standard_normal((n_comp, hd)).astype(np.float32)
+    sk = rng.standard_normal(heads).astype(np.float32)
+    got = _order_free_attention(ctx, dev, q, win, comp, sk, inv, nope, pairs, 777)[False].astype(np.float64)
+    u, keys, q64 = 2.0 ** -24, np.concatenate([win, comp]).astype(np.float64), q.astype(np.float64)
+    sc = q64 @ keys.T * hd ** -0.5
+    mx = sc.max(1, keepdims=True)
+    w = np.exp(sc - mx)
+    w /= w.sum(1, keepdims=True) + np.exp(sk[:, None] - mx)
+    d = ((hd + 2) * u * (np.abs(q64) @ np.abs(keys).T) * hd ** -0.5).max(1, keepdims=True)
+    tol = (4 * d + 2 * (len(keys) + 18) * u) * (w @ np.abs(keys)) + 1e-37
+    want = w @ keys
+    ang = (np.float32(777) * inv[:pairs]).astype(np.float64)
+    r = slice(nope, nope + 2 * pairs)
+    e, o = want[:, r][:, ::2].copy(), want[:, r][:, 1::2].copy()
+    want[:, r][:, ::2], want[:, r][:, 1::2] = e * np.cos(ang) + o * np.sin(ang), o * np.cos(ang) - e * np.sin(ang)
+    pair = tol[:, r][:, ::2] + tol[:, r][:, 1::2]
+    tol[:, r][:, ::2], tol[:, r][:, 1::2] = pair, pair
+    assert np.all(np.abs(got - want) <= tol), float((np.abs(got - want) / tol).max())
+
+
+def test_window_attention_order_free_infinite_scores(ctx, dev):
+    """Tiles whose scores are all -inf weigh nothing beside a finite one, a
+    head with only such scores is NaN, and a NaN score makes its head NaN, as
+    in the ordered kernels."""
+    rng = np.random.default_rng(3)
+    q = rng.standard_normal((33, 64)).astype(np.float32)
+    keys = rng.standard_normal((96, 64)).astype(np.float32)
+    q[:, 5] = 1e20
+    q[7, 5] = -1e20   # +inf scores
+    keys[:, 5] = 0.0
+    keys[:64, 5] = -1e20  # two tiles of -inf
+    sk, inv = np.zeros(33, np.float32), np.ones(1, np.float32)
+    o = _order_free_attention(ctx, dev, q, keys, keys[:0], sk, inv, 64, 0, 3)
+    assert np.array_equal(np.isnan(o[True]), np.isnan(o[False])) and np.isnan(o[False][7]).all()
+    live = ~np.isnan(o[True])
+    assert live.any() and np.allclose(o[True][live], o[False][live], rtol=1e-4, atol=1e-5)
+    keys[64:, 5] = -1e20
+    o = _order_free_attention(ctx, dev, q, keys, keys[:0], sk, inv, 64, 0, 3)
+    assert np.isnan(o[True]).all() and np.isnan(o[False]).all()
+
+
 # ---------------------------------------------------------------- the layer
 HEADS, NOPE, ROPE, Q_LORA, GROUPS, O_LORA = 64, 448, 64, 1024, 8, 1024
 HEAD_DIM = NOPE + ROPE

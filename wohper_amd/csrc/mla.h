@@ -252,6 +252,7 @@ struct wh_attn_args {
     // 0), compressed rows bcomp[z] (bncomp[z] of them)
     uint32_t nb, q_ld, scores_ld, wlen;
     uint32_t max_keys;     // the longest key list
+    float* tile_max;       // attn_mx.h: [nb][heads][64]
     uint32_t wts_ld;       // k_attn_combine: floats per head of its dynamic LDS (>= every n_keys)
     uint32_t bpos[WH_POS_BATCH];
     uint32_t bncomp[WH_POS_BATCH];

@@ -22,6 +22,7 @@
 #include "kernels.h"
 #include "mhc.h"
 #include "mla.h"
+#include "attn_mx.h"
 #include "moe_batch.h"
 #include "moe_px.h"
 #include "moe_tok.h"
@@ -297,6 +298,7 @@ struct wh_ctx {
     uint32_t fp8_mm_min = 4;                // multi-input FP8 GEMVs with this many inputs use MFMA
     Scratch fp8mm_ws, fp8mm_cnt;            // their partial tiles and arrival counters
     Scratch moe_dyn;                        // a device route list resolved for the experts (wh_moe_dyn)
+    Scratch attn_max;                       // attn_mx.h: the score tiles' maxima, of a fixed size
     Scratch layer;                          // the decode layer's state and activations between its steps
     bool exact = true;                      // routed experts in the reference's summation order
     int token_kernels = 1;                  // MFMA token kernels: bit 0 gate/up, bit 1 down on k_*_tok (else k_*_px)
@@ -316,7 +318,7 @@ struct wh_ctx {
     hipStream_t base_stream = nullptr, cap_stream = nullptr;
     std::vector<Scratch*> scratch() {
         return {&x_in, &y_out, &h, &ybuf, &cnt_y, &tmp, &batch, &routes, &bout, &gu, &relayout, &rtr, &rtr_cnt,
-                &mla, &hcs, &fp8mm_ws, &fp8mm_cnt, &moe_dyn, &layer};
+                &mla, &hcs, &fp8mm_ws, &fp8mm_cnt, &moe_dyn, &attn_max, &layer};
     }
 };
 
@@ -2028,6 +2030,8 @@ int wh_init(int device, wh_ctx** out) {
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->status_host, sizeof(uint32_t), hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreate(&c->timer[0]);
     if (e == hipSuccess) e = hipEventCreate(&c->timer[1]);
+    if (e == hipSuccess)
+        e = c->attn_max.ensure((size_t)WH_POS_BATCH * WH_ATTN_MX_HEADS * WH_ATTN_MX_TILES * sizeof(float), false);
     if (e != hipSuccess) {
         delete c;
         return hip_status(e);
@@ -3791,12 +3795,30 @@ wh_rowpost_args rowpost_args(const float* x, float* out, size_t rows, size_t n, 
     return a;
 }
 
+void attn_mx_launch(wh_ctx* c, const wh_attn_args& a, unsigned nb) {
+    const unsigned tiles = (a.max_keys + WH_ATTN_MX_KEYS - 1) / WH_ATTN_MX_KEYS;
+    const unsigned g16 = (a.heads + 15) / 16, g32 = (a.heads + 31) / 32;
+    if ((size_t)tiles * g32 * nb >= 512) k_attn_scores_mx<2><<<dim3(tiles, g32, nb), 256, 0, c->stream>>>(a);
+    else k_attn_scores_mx<1><<<dim3(tiles, g16, nb), 256, 0, c->stream>>>(a);
+    if ((size_t)(a.head_dim / 64) * g32 * nb >= 256)
+        k_attn_weighted_mx<2, 4><<<dim3(a.head_dim / 64, g32, nb), 256, 0, c->stream>>>(a);
+    else k_attn_weighted_mx<1, 1><<<dim3(a.head_dim / 16, g16, nb), 256, 0, c->stream>>>(a);
+}
+
 // The window softmax of one position, or of args.nb.
 int attn_launch(wh_ctx* c, const wh_attn_args& args) {
     wh_attn_args a = args;
     const unsigned nb = a.nb ? a.nb : 1u;
     if (!a.nb) a.max_keys = a.n_win + a.n_comp;
     const unsigned nk = a.max_keys, blocks = a.head_dim / 64;
+    // exact numerics off: the sums on matrix instructions (attn_mx.h), which
+    // read q and the keys 16 bytes at a time
+    if (!c->exact && a.heads <= WH_ATTN_MX_HEADS && !((uintptr_t)a.q & 15)) {
+        a.tile_max = c->attn_max.as<float>();
+        attn_mx_launch(c, a, nb);
+        WH_HIP(hipGetLastError());
+        return WH_OK;
+    }
     a.wts_ld = (nk + 3) & ~3u;
     // heads per wave: four share each key's way through LDS once that leaves
     // two waves for every SIMD (2048), else as many waves as there are heads
