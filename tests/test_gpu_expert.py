@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import wohper_amd
+from test_gpu_mla import Dev
 from wohper_amd import workloads as wl
 
 pytestmark = pytest.mark.gpu
@@ -51,6 +52,34 @@ def test_act_quant_midpoints_and_known_answers(ctx, oracle):
     assert np.array_equal(bits(ctx.act_quant_dequant(x, 64)), bits(oracle.act_quant(x, 64)))
     k = KATS["act_quant_representable"]
     assert np.all(np.abs(ctx.act_quant_dequant(np.array(k["values"], np.float32), k["block"]) - k["expected"]) < k["tol"])
+
+
+@pytest.mark.parametrize("blocks", [1, 3, 15, 16, 17, 520])
+@pytest.mark.parametrize("shift", [0, 4, 1])
+def test_act_quant64_device(ctx, oracle, blocks, shift):
+    """Whole blocks of 64 on the device, 16 lanes a block, and the general
+    kernel where they do not start on 16 bytes (shift 1): the oracle's bits,
+    infinite and NaN values among them, and nothing written beside them."""
+    rng = np.random.default_rng(blocks)
+    x = (rng.standard_normal(64 * blocks) * np.exp2(rng.integers(-30, 30, blocks)).repeat(64)).astype(np.float32)
+    x[0] = 0.0
+    if blocks > 2:
+        x[70], x[140], x[150] = np.inf, np.nan, -0.0
+    buf = np.full(x.size + 8, 7.0, np.float32)
+    buf[shift:shift + x.size] = x
+    dev = Dev(ctx)
+    try:
+        p = dev.put(buf)
+        ctx.act_quant_dequant_async(p + 4 * shift, x.size, 64)
+        ctx.synchronize()
+        got = dev.get(p, buf.size)
+    finally:
+        dev.free()
+    with np.errstate(all="ignore"):
+        want = oracle.act_quant(x, 64)
+    g, same = got[shift:shift + x.size], ~np.isnan(want)
+    assert np.array_equal(bits(g[same]), bits(want[same])) and np.all(np.isnan(g[~same]))
+    assert np.all(got[:shift] == 7.0) and np.all(got[shift + x.size:] == 7.0)
 
 
 def test_tiny_expert_known_answer(ctx, oracle):

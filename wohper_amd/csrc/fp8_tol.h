@@ -18,11 +18,6 @@
 #pragma once
 #include "kernels.h"
 
-template <int kCtrl>
-__device__ __forceinline__ float wh_dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kCtrl, 0xF, 0xF, false));
-}
-
 // One halving step of a wave sum over lane bit kB (32, 16, 8, 4, 2, 1):
 // every lane holds kN partial sums v[0..kN); lanes with bit kB clear keep
 // sums [0, kN/2), the others [kN/2, kN), each adding the copy of a partner

@@ -126,6 +126,11 @@ __device__ __forceinline__ float wh_hsum8(float v) {
     return p2 + wh_dpp_row_shl4(p2);
 }
 
+template <int kCtrl>
+__device__ __forceinline__ float wh_dpp_f(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kCtrl, 0xF, 0xF, false));
+}
+
 __device__ __forceinline__ float wh_wave_max(float v) {
     for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
     return v;

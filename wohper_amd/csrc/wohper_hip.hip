@@ -1135,6 +1135,17 @@ int moe_shapes(const ExpertView* ev, size_t n, bool* fast) {
     return WH_OK;
 }
 
+// The act-quant of n values in place.  Blocks of 64 that are whole and start
+// on 16 bytes (every activation of the layers) take the kernel of 16 lanes a
+// block; other block sizes, a last partial block and odd pointers the general
+// one.
+void act_quant_launch(wh_ctx* c, float* v, size_t n, size_t block) {
+    if (block == 64 && n % 64 == 0 && !((uintptr_t)v & 15))
+        k_act_quant64_inplace<<<(unsigned)((n + 1023) / 1024), 256, 0, c->stream>>>(v, (uint32_t)n);
+    else
+        k_act_quant_inplace<<<(unsigned)((n + block - 1) / block), 256, 0, c->stream>>>(v, (uint32_t)n, (uint32_t)block);
+}
+
 // Routed experts for n_tokens rows of x (all with the same route list).
 // x_dev: device input (f32 or bf16).  out_dev: n_tokens x hidden f32.
 // ev[0..n): the experts; with has_shared the last one is the shared expert
@@ -1164,11 +1175,11 @@ int moe_forward(wh_ctx* c, const ExpertView* ev, const float* route_w, size_t n,
         const float* xt = (const float*)x_dev + tok * hidden;
         for (size_t i = 0; i < n; ++i) {
             WH_HIP(hipMemcpyAsync(xq, xt, hidden * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-            k_act_quant_inplace<<<(unsigned)((hidden + 63) / 64), 256, 0, c->stream>>>(xq, (uint32_t)hidden, 64);
+            act_quant_launch(c, xq, hidden, 64);
             WH_TRY(launch_fp4(c, *ev[i].w1, xq, g));
             WH_TRY(launch_fp4(c, *ev[i].w3, xq, u));
             k_swiglu_generic<<<(unsigned)((inter + 255) / 256), 256, 0, c->stream>>>(g, u, hh, (uint32_t)inter, c->status);
-            k_act_quant_inplace<<<(unsigned)((inter + 63) / 64), 256, 0, c->stream>>>(hh, (uint32_t)inter, 64);
+            act_quant_launch(c, hh, inter, 64);
             WH_TRY(launch_fp4(c, *ev[i].w2, hh, ys + i * osz));
         }
         k_combine_generic<<<(unsigned)((osz + 255) / 256), 256, 0, c->stream>>>(
@@ -2980,8 +2991,7 @@ int wh_act_quant_dequant(wh_ctx* c, float* values, size_t n, size_t block) {
     WH_HIP(hipSetDevice(c->device));
     WH_HIP(c->x_in.ensure(n * sizeof(float), false));
     WH_HIP(hipMemcpyAsync(c->x_in.p, values, n * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    k_act_quant_inplace<<<(unsigned)((n + block - 1) / block), 256, 0, c->stream>>>(
-        c->x_in.as<float>(), (uint32_t)n, (uint32_t)block);
+    act_quant_launch(c, c->x_in.as<float>(), n, block);
     WH_HIP(hipGetLastError());
     WH_HIP(hipMemcpyAsync(values, c->x_in.p, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     WH_HIP(hipStreamSynchronize(c->stream));
@@ -3415,11 +3425,11 @@ int fp8_shared_launch(wh_ctx* c, const Tensor& w1, const Tensor& w3, const Tenso
     float* up = gate + inter;
     float* h = up + inter;
     WH_HIP(hipMemcpyAsync(xq, x_dev, hidden * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-    k_act_quant_inplace<<<(unsigned)((hidden + 63) / 64), 256, 0, c->stream>>>(xq, (uint32_t)hidden, 64);
+    act_quant_launch(c, xq, hidden, 64);
     WH_TRY(launch_fp8(c, w1, 0, inter, xq, gate, 1, hidden, inter));
     WH_TRY(launch_fp8(c, w3, 0, inter, xq, up, 1, hidden, inter));
     k_swiglu_generic<<<(unsigned)((inter + 255) / 256), 256, 0, c->stream>>>(gate, up, h, (uint32_t)inter, c->status);
-    k_act_quant_inplace<<<(unsigned)((inter + 63) / 64), 256, 0, c->stream>>>(h, (uint32_t)inter, 64);
+    act_quant_launch(c, h, inter, 64);
     WH_TRY(launch_fp8(c, w2, 0, w2.rows, h, y_dev, 1, inter, w2.rows));
     WH_HIP(hipGetLastError());
     return WH_OK;
@@ -3918,8 +3928,7 @@ int wh_act_quant_dequant_async(wh_ctx* c, float* values_dev, size_t n, size_t bl
     if (n > 0xffffffffu || (n + block - 1) / block > 0x7fffffffu) return WH_UNSUPPORTED;
     std::lock_guard<std::recursive_mutex> lk(c->mu);
     WH_HIP(hipSetDevice(c->device));
-    k_act_quant_inplace<<<(unsigned)((n + block - 1) / block), 256, 0, c->stream>>>(values_dev, (uint32_t)n,
-                                                                                     (uint32_t)block);
+    act_quant_launch(c, values_dev, n, block);
     WH_HIP(hipGetLastError());
     return WH_OK;
 }
@@ -4088,7 +4097,7 @@ static int mla_decode_impl(wh_ctx* c, const wh_mla_layer* L, size_t token_pos, c
     w.scale = powf((float)head_dim, -0.5f);
     WH_TRY(attn_launch(c, w));
     // grouped output projection (E/compute.rs:4222-4270)
-    k_act_quant_inplace<<<(unsigned)((q_full + 63) / 64), 256, 0, c->stream>>>(at, (uint32_t)q_full, 64);
+    act_quant_launch(c, at, q_full, 64);
     if (fp8_split_k(*wo_a) && is_pow2(o_lora) && o_lora >= WH_FP8_SK_ROWS && group_in <= 0xffffffffu) {
         WH_TRY(launch_fp8(c, *wo_a, 0, o_mid, at, om, 1, group_in, o_mid, o_lora, group_in));
     } else {
@@ -4096,7 +4105,7 @@ static int mla_decode_impl(wh_ctx* c, const wh_mla_layer* L, size_t token_pos, c
             WH_TRY(launch_fp8(c, *wo_a, g * o_lora, (g + 1) * o_lora, at + g * group_in, om + g * o_lora, 1,
                               group_in, o_lora));
     }
-    k_act_quant_inplace<<<(unsigned)((o_mid + 63) / 64), 256, 0, c->stream>>>(om, (uint32_t)o_mid, 64);
+    act_quant_launch(c, om, o_mid, 64);
     WH_TRY(launch_fp8(c, *wo_b, 0, hidden, om, hidden_dev, 1, o_mid, hidden));
     WH_HIP(hipGetLastError());
     return WH_OK;
@@ -4252,16 +4261,13 @@ static int mla_decode_batch_impl(wh_ctx* c, const wh_mla_layer* L, const size_t*
     }
     // o path (E/compute.rs:4582-4631): act-quant per position, wo_a per
     // output group over all positions, act-quant, wo_b over all positions
-    k_act_quant_inplace<<<(unsigned)((npos * q_full + 63) / 64), 256, 0, c->stream>>>(at, (uint32_t)(npos * q_full),
-                                                                                     64);
+    act_quant_launch(c, at, npos * q_full, 64);
     WH_TRY(wh_fp8_gemv_multi_groups_async(c, L->wo_a, 0, o_mid, o_lora, at, group_in, npos, q_full, om, o_mid));
     if (o_mid % 64 == 0)  // (q_full is: head_dim % 64 == 0) the 64-blocks stay inside their position
-        k_act_quant_inplace<<<(unsigned)((npos * o_mid + 63) / 64), 256, 0, c->stream>>>(om, (uint32_t)(npos * o_mid),
-                                                                                        64);
+        act_quant_launch(c, om, npos * o_mid, 64);
     else
         for (size_t i = 0; i < npos; ++i)
-            k_act_quant_inplace<<<(unsigned)((o_mid + 63) / 64), 256, 0, c->stream>>>(om + i * o_mid, (uint32_t)o_mid,
-                                                                                     64);
+            act_quant_launch(c, om + i * o_mid, o_mid, 64);
     WH_TRY(wh_fp8_gemv_multi_async(c, L->wo_b, 0, hidden, om, npos, o_mid, hidden_dev, hidden));
     WH_HIP(hipGetLastError());
     return WH_OK;
