@@ -87,6 +87,56 @@ def test_decode_layer_batch_order_free(ctx, oracle, dev):
         ctx.release(t)
 
 
+@pytest.mark.parametrize("n", [5, 16, 17, 33, 131])
+def test_decode_layer_batch_matches_small(ctx, oracle, dev, n):
+    """Exact numerics: n positions in one call against calls of at most four,
+    bit for bit: the projections and the router of 16 inputs on matrix
+    instructions with a partial last tile, and more positions than one launch
+    of the window attention takes."""
+    ctx.set_exact_numerics(True)
+    L, _, handles = _setup(ctx, oracle, dev)
+    cap, ld = n + 3, HEAD_DIM
+    rng = np.random.default_rng(n)
+    kv0 = np.zeros((cap, ld), np.float32)
+    kv0[:3] = (rng.standard_normal((3, ld)) * 0.3).astype(np.float32)
+    positions = list(range(3, 3 + n))
+    h0 = (rng.standard_normal((n, HC * wl.HIDDEN)) * 0.5).astype(np.float32)
+    got, got_kv = _run(ctx, dev, L, h0, positions, kv0, ld)
+    want, want_kv = np.empty_like(got), kv0
+    for i in range(0, n, 4):
+        want[i:i + 4], want_kv = _run(ctx, dev, L, h0[i:i + 4], positions[i:i + 4], want_kv, ld)
+    assert np.array_equal(bits(got_kv), bits(want_kv))
+    for i in range(n):
+        assert np.array_equal(bits(got[i]), bits(want[i])), (i, int(np.count_nonzero(bits(got[i]) != bits(want[i]))))
+    for t in handles.values():
+        ctx.release(t)
+
+
+def test_decode_layer_batch_order_free_many(ctx, oracle, dev):
+    """Exact numerics off, 33 positions in one call (hc_pre's sums of four
+    streams a workgroup, a partial last one) against calls of at most 8: the
+    bounds of the test above against the exact batch, for the same reasons."""
+    L, _, handles = _setup(ctx, oracle, dev)
+    n, ld = 33, HEAD_DIM
+    rng = np.random.default_rng(23)
+    kv0 = (rng.standard_normal((n + 2, ld)) * 0.3).astype(np.float32)
+    positions = list(range(2, 2 + n))
+    h0 = (rng.standard_normal((n, HC * wl.HIDDEN)) * 0.5).astype(np.float32)
+    ctx.set_exact_numerics(False)
+    got, _ = _run(ctx, dev, L, h0, positions, kv0, ld)
+    want = np.empty_like(got)
+    kv = kv0
+    for i in range(0, n, 8):
+        want[i:i + 8], kv = _run(ctx, dev, L, h0[i:i + 8], positions[i:i + 8], kv, ld)
+    assert np.all(np.isfinite(got))
+    rel = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    print("per-position ||diff|| / ||value||:", np.array2string(rel, precision=6))
+    assert float(rel.max()) <= 0.1
+    assert float(np.median(rel)) <= 3e-2
+    for t in handles.values():
+        ctx.release(t)
+
+
 def test_decode_layer_batch_errors(ctx, oracle, dev):
     L, want, handles = _setup(ctx, oracle, dev)
     cap, ld = 8, HEAD_DIM

@@ -4358,6 +4358,10 @@ int hc_pre_launch(wh_ctx* c, const float* fn_dev, const float* scale_dev, const 
         else if (a.hc_dim <= 4096) chains(integral_constant<int, 128>(), integral_constant<int, 32>());
         else if (a.hc_dim <= 8192) chains(integral_constant<int, 128>(), integral_constant<int, 64>());
         else chains(integral_constant<int, 256>(), integral_constant<int, 64>());
+    } else if (npos >= 32 && a.hc_dim == WH_HC_PARTS * 1024) {
+        // four streams a workgroup: 16 streams 5.6 us before, 7.7 so; 32
+        // streams 9.5 and 7.8, 64 15.9 and 8.5
+        k_hc_partials_multi<4><<<dim3(WH_HC_PARTS, (z + 3) / 4), 256, 0, c->stream>>>(a, z);
     } else {
         k_hc_partials<<<dim3(WH_HC_PARTS, a.mix_hc + 1, z), 256, 0, c->stream>>>(a);
     }
