@@ -632,6 +632,138 @@ __global__ void __launch_bounds__(64) k_router_bf16(const uint16_t* __restrict__
     if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The one-launch router's gate for many inputs (grid (rows / 16, ceil(n / 16)),
+// 256 threads, cols % 1024 == 0, rows % 16 == 0): scores and selection keys of
+// 16 rows x 16 inputs, published as k_router_bf16 publishes them, for
+// k_router_select_lists.  The gate runs on v_mfma_f32_16x16x1_4b_f32, whose
+// four blocks of 16 x 16 outputs take one product a step, an FMA rounded once:
+// a block carries one of the 16 AVX accumulator chains of dot_bf16_row, and
+// the four waves the four chains each, so the logits are k_router_bf16's bits.
+//
+// Why: there every 4 rows of every input were a workgroup that fetched the
+// input and its rows anew (400 MB from L2 for 128 inputs).  128 inputs 64.5 us,
+// now 16.0 us and 4.7 us for the selection's launch.
+#define WH_ROUTER_MM_GROUPS 4u  // 128-column blocks a chunk of x in LDS
+typedef float wh_router_f16 __attribute__((ext_vector_type(16)));
+__global__ void __launch_bounds__(256) k_router_mm(const uint16_t* __restrict__ w, const float* __restrict__ x,
+                                                   uint32_t cols, wh_router_sel a, uint32_t n_in, uint32_t x_ld,
+                                                   uint32_t pub_ld) {
+    constexpr uint32_t kG = WH_ROUTER_MM_GROUPS, kChunk = 128 * kG;
+    constexpr uint32_t kLd = kChunk + 4;  // floats per input: 16 inputs' 16-byte reads fall on 16 bank groups
+    constexpr int kUnits = 16 * kChunk / 16 / 256;
+    __shared__ __align__(16) float xs[2][16 * kLd];
+    __shared__ uint64_t exp_tab[WH_EXP_TAB_LEN];
+    const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63, q = lane >> 4, col = lane & 15;
+    const uint32_t row0 = blockIdx.x * 16, i0 = blockIdx.y * 16, n_here = min(16u, n_in - i0);
+    const uint32_t n_chunks = cols / kChunk;
+    if (t < WH_EXP_TAB_LEN) exp_tab[t] = kExpTab[t];
+    // A: block q is chain 4 wave + q of row `col`; a chain's eight values of a
+    // 128-column block are 16 contiguous bytes
+    const uint4* wp = (const uint4*)(w + (size_t)(row0 + col) * cols) + 4 * wave + q;
+    uint4 wv[2][kG];
+    auto load_w = [&](int b, uint32_t chunk) {
+        const uint32_t g0 = min(chunk, n_chunks - 1) * kG;
+#pragma unroll
+        for (uint32_t g = 0; g < kG; ++g) wv[b][g] = wp[16 * (g0 + g)];
+    };
+    // x: unit u is 16 columns of an input, one value for each chain
+    const uint32_t uc = t & 7, un = (t >> 3) & 15, ug = t >> 7;
+    const float* xp = x + (size_t)(i0 + min(un, n_here - 1)) * x_ld + 128 * ug + 16 * uc;
+    float4 xr[2][kUnits][4];
+    auto load_x = [&](int b, uint32_t chunk) {
+        const float* p = xp + (size_t)min(chunk, n_chunks - 1) * kChunk;
+#pragma unroll
+        for (int k = 0; k < kUnits; ++k)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) xr[b][k][j] = *(const float4*)(p + 256 * k + 4 * j);
+    };
+    auto store_x = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < kUnits; ++k) {
+            float* d = xs[b] + un * kLd + 128 * (ug + 2 * k) + uc;
+#pragma unroll
+            for (int o = 0; o < 16; ++o) d[o * 8] = wh_f4_get(xr[b][k][o >> 2], o & 3);
+        }
+    };
+    wh_router_f16 d;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) d[r] = 0.0f;
+    auto chunk_mm = [&](int b) {
+#pragma unroll
+        for (uint32_t g = 0; g < kG; ++g) {
+            const float4* p = (const float4*)(xs[b] + col * kLd + 128 * g + (4 * wave + q) * 8);
+            const float4 x0 = p[0], x1 = p[1];
+            const uint4 w4 = wv[b][g];
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_lo(w4.x), x0.x, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_hi(w4.x), x0.y, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_lo(w4.y), x0.z, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_hi(w4.y), x0.w, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_lo(w4.z), x1.x, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_hi(w4.z), x1.y, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_lo(w4.w), x1.z, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x1f32(wh_bf16_hi(w4.w), x1.w, d, 0, 0, 0);
+        }
+    };
+    // chunk k in buffer k % 2; its weights and x are requested two chunks ahead
+    // (the loop has no branch: where paths met, every load was waited for)
+    load_x(0, 0);
+    load_w(0, 0);
+    load_x(1, 1);
+    load_w(1, 1);
+    store_x(0);
+    __syncthreads();
+    auto step = [&](uint32_t k, int b) {
+        load_x(b, k + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        chunk_mm(b);
+        load_w(b, k + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        store_x(b ^ 1);
+        __syncthreads();
+    };
+    for (uint32_t k = 0; k < n_chunks; k += 2) {
+        step(k, 0);
+        step(k + 1, 1);
+    }
+    // acc0 + acc1 of each AVX lane, then hsum256's pairs; block b's
+    // D[4 (lane / 16) + r][lane % 16] in d[4 b + r], red[chain][input][row]
+    float* red = xs[0];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[((4 * wave + b) * 16 + col) * 17 + 4 * q + r] = d[4 * b + r];
+    __syncthreads();
+    const uint32_t n = t >> 4, j = t & 3, row = row0 + (t & 15);
+    float s[8];
+#pragma unroll
+    for (int l = 0; l < 8; ++l) s[l] = red[(l * 16 + n) * 17 + (t & 15)] + red[((l + 8) * 16 + n) * 17 + (t & 15)];
+    const float v = (((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))) + 0.0f;
+    // four rows in selection order, as in k_router_bf16
+    const float score = a.math ? wh_sqrt_softplus(v, exp_tab) : v;
+    const int32_t key = wh_total_key(a.math && a.bias ? score + a.bias[row] : score);
+    uint32_t rank = 0;
+#pragma unroll
+    for (uint32_t o = 0; o < 4; ++o) {
+        const int32_t ko = __shfl(key, (int)((lane & ~3u) + o), 64);
+        rank += (ko > key || (ko == key && o < j)) ? 1u : 0u;
+    }
+    if (n >= n_here) return;
+    float* pub = const_cast<float*>(a.logits) + (size_t)(i0 + n) * pub_ld;
+    const uint32_t at = row - j + rank;
+    ((uint64_t*)pub)[at] = ((uint64_t)(uint32_t)key << 32) | __float_as_uint(score);
+    ((uint32_t*)(pub + 2 * a.rows))[at] = row;
+}
+
+// The selection after k_router_mm: one wave per input.
+__global__ void __launch_bounds__(64) k_router_select_lists(wh_router_sel a, uint32_t pub_ld) {
+    const uint32_t z = blockIdx.x;
+    a.logits += (size_t)z * pub_ld;
+    a.out_ids += (size_t)z * a.active;
+    a.out_scores += (size_t)z * a.active;
+    a.out_count += z;
+    wh_router_select_sorted<false>(a);
+}
+
 // Test support: fn 4 sqrt_softplus(x), fn 5 log1pf(x) (x >= 0), fn 6 expf(x)
 // over the whole float line.
 __global__ void k_debug_eval_router(int fn, const float* __restrict__ in, float* __restrict__ out, uint32_t n) {

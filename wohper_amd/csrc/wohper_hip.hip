@@ -1929,8 +1929,17 @@ int route_batch(wh_ctx* c, uint32_t layer, const float* x, size_t x_ld, size_t h
     sa.out_scores = scores;
     sa.out_count = count;
     sa.sorted = 1;
-    k_router_bf16<false><<<dim3((unsigned)(rt.rows / 4), (unsigned)npos), 64, rt.cols * sizeof(float), c->stream>>>(
-        rt.bf16, x, (uint32_t)rt.cols, sa, c->rtr_cnt.as<uint32_t>(), (uint32_t)x_ld, (uint32_t)pub_ld);
+    // the gate on matrix instructions from 24 inputs on (16 inputs 22.1
+    // us before, 20.1 so with its second launch, 32 inputs 31.4 and 20.1, 128
+    // inputs 64.5 and 20.7; its time hardly depends on them)
+    if (npos >= 24 && rt.rows % 16 == 0 && rt.cols % (256 * WH_ROUTER_MM_GROUPS) == 0) {
+        k_router_mm<<<dim3((unsigned)(rt.rows / 16), (unsigned)((npos + 15) / 16)), 256, 0, c->stream>>>(
+            rt.bf16, x, (uint32_t)rt.cols, sa, (uint32_t)npos, (uint32_t)x_ld, (uint32_t)pub_ld);
+        k_router_select_lists<<<(unsigned)npos, 64, 0, c->stream>>>(sa, (uint32_t)pub_ld);
+    } else {
+        k_router_bf16<false><<<dim3((unsigned)(rt.rows / 4), (unsigned)npos), 64, rt.cols * sizeof(float), c->stream>>>(
+            rt.bf16, x, (uint32_t)rt.cols, sa, c->rtr_cnt.as<uint32_t>(), (uint32_t)x_ld, (uint32_t)pub_ld);
+    }
     WH_HIP(hipGetLastError());
     return WH_OK;
 }
