@@ -230,6 +230,16 @@ def test_window_attention_order_free(ctx, dev, heads, hd, nope, pairs, n_win, n_
     assert np.all(np.abs(got - want) <= tol), float((np.abs(got - want) / tol).max())
 
 
+@pytest.mark.parametrize("heads", [225, 256])
+@pytest.mark.parametrize("hd,nope,pairs", [(64, 0, 32), (192, 128, 32), (512, 448, 32)])
+@pytest.mark.parametrize("n_comp", [1857, 1888, 1889, 1920])
+def test_window_attention_order_free_wide(ctx, dev, heads, hd, nope, pairs, n_comp):
+    """32 heads x 64 keys a workgroup (from 256 of those on): one, odd and even
+    numbers of dim tiles, a partial tile of heads, key lists that end in either
+    half of a tile; the bound of the test above."""
+    test_window_attention_order_free(ctx, dev, heads, hd, nope, pairs, 128, n_comp)
+
+
 def test_window_attention_order_free_infinite_scores(ctx, dev):
     """Tiles whose scores are all -inf weigh nothing beside a finite one, a
     head with only such scores is NaN, and a NaN score makes its head NaN, as

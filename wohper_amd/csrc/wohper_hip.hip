@@ -3817,7 +3817,8 @@ wh_rowpost_args rowpost_args(const float* x, float* out, size_t rows, size_t n, 
 void attn_mx_launch(wh_ctx* c, const wh_attn_args& a, unsigned nb) {
     const unsigned tiles = (a.max_keys + WH_ATTN_MX_KEYS - 1) / WH_ATTN_MX_KEYS;
     const unsigned g16 = (a.heads + 15) / 16, g32 = (a.heads + 31) / 32;
-    if ((size_t)tiles * g32 * nb >= 512) k_attn_scores_mx<2><<<dim3(tiles, g32, nb), 256, 0, c->stream>>>(a);
+    const unsigned wide = (a.max_keys + 63) / 64;
+    if ((size_t)wide * g32 * nb >= 256) k_attn_scores_mx_tile<<<dim3(wide, g32, nb), 256, 0, c->stream>>>(a);
     else k_attn_scores_mx<1><<<dim3(tiles, g16, nb), 256, 0, c->stream>>>(a);
     if ((size_t)(a.head_dim / 64) * g32 * nb >= 256)
         k_attn_weighted_mx<2, 4><<<dim3(a.head_dim / 64, g32, nb), 256, 0, c->stream>>>(a);
