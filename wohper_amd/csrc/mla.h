@@ -231,6 +231,46 @@ __global__ void __launch_bounds__(kT) k_rowpost(wh_rowpost_args a) {
     for (uint32_t i = t; i < n; i += kT) out[i] = v[i];
 }
 
+// k_rowpost for rows of 512 with the norm (no weights, the sum in the fixed
+// tree) and RoPE only: the heads of q with exact numerics off.  One wave a
+// row, no LDS and no barrier: lane L holds elements 64 k + L, so the tree's
+// four waves are four butterflies of this one and a rotated pair sits in
+// neighbouring lanes.  The same bits.  Bound by memory: 8192 heads, 33.6 MB
+// both ways, 11.0 us; with a workgroup a row, five barriers and a 16 KB
+// copy of it in LDS, 37.4 us (in four launches).  blockDim / 64 rows a workgroup.
+__global__ void __launch_bounds__(256) k_rowpost_heads(wh_rowpost_args a) {
+    const uint32_t lane = threadIdx.x & 63, row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (row >= a.rows) return;  // a whole wave
+    const float* x = a.x + (size_t)row * a.ld_in + lane;
+    float xv[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) xv[k] = x[64 * k];
+    float s[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) s[w] = (0.0f + xv[w] * xv[w]) + xv[w + 4] * xv[w + 4];
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s[w] = s[w] + __shfl_xor(s[w], off, 64);
+    const float inv = 1.0f / sqrtf((((s[0] + s[1]) + s[2]) + s[3]) / 512.0f + 1.0e-6f);
+    const float pos = (float)(a.rows_per_pos ? a.bpos[row / a.rows_per_pos] : a.position);
+    float* out = a.out + (size_t)row * a.ld_out + lane;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        float y = xv[k] * inv;
+        if (64u * k + 63 >= a.rope_off && 64u * k < a.rope_off + 2 * a.pairs) {  // uniform
+            const uint32_t i = 64 * k + lane, p = (i - a.rope_off) >> 1;
+            const bool on = i >= a.rope_off && p < a.pairs;
+            const float ang = pos * (on ? a.inv_freqs[p] : 0.0f);
+            float sn = wh_sincosf_glibc(ang, 0);
+            const float cs = wh_sincosf_glibc(ang, 1);
+            if (a.inverse) sn = -sn;
+            const float other = __shfl_xor(y, 1, 64);
+            if (on) y = (i & 1) ? other * sn + y * cs : y * cs - other * sn;
+        }
+        out[64 * k] = y;
+    }
+}
+
 // --------------------------------------------------------- window softmax
 // Keys of one decode position: the window rows (the KV cache at positions
 // [window_start, token_pos], row stride win_ld) then the visible compressed
