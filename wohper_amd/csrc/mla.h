@@ -17,7 +17,7 @@
 #define WH_ROWPOST_MAX 4096u     // values per row of k_rowpost
 #define WH_ATTN_MAX_KEYS 2048u   // window + compressed keys per head
 #define WH_ATTN_MAX_HEAD_DIM 1024u
-#define WH_POS_BATCH 32u         // positions per batched launch of k_rowpost / the attention
+#define WH_POS_BATCH 128u        // positions per batched launch of k_rowpost / the attention
 
 __device__ __forceinline__ float wh_bf16_value(uint16_t raw) { return __uint_as_float((uint32_t)raw << 16); }
 
@@ -70,20 +70,20 @@ struct wh_rowpost_args {
     uint32_t hc, hc_stride;
 };
 
-// kT threads per row (256, or 1024 for a lone row); each thread's values
+// One row by kT threads (256, or 1024 for a lone row); each thread's values
 // and norm weights are loaded up front.
 template <int kT>
-__global__ void __launch_bounds__(kT) k_rowpost(wh_rowpost_args a) {
+__device__ __forceinline__ void wh_rowpost_row(const wh_rowpost_args& a, uint32_t row) {
     constexpr int kPer = WH_ROWPOST_MAX / kT;  // values per thread at most
     constexpr int kW = kT / 64;                // waves
     __shared__ __align__(16) float v[WH_ROWPOST_MAX];
     __shared__ float inv_s;
     const uint32_t t = threadIdx.x, n = a.n;
-    const float* x = a.x + (size_t)blockIdx.x * a.ld_in;
+    const float* x = a.x + (size_t)row * a.ld_in;
     uint32_t position = a.position;
-    size_t orow = blockIdx.x;
+    size_t orow = row;
     if (a.rows_per_pos) {
-        position = a.bpos[blockIdx.x / a.rows_per_pos];
+        position = a.bpos[row / a.rows_per_pos];
         if (a.out_at_pos) orow = position;
     }
     float xv[kPer], wv[kPer];
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(kT) k_rowpost(wh_rowpost_args a) {
     uint32_t wr[kPer];
     if (a.hc == 4) {
         // the four copies' loads issued together, then the reference's sum
-        const float* pre = a.hc_pre + (size_t)blockIdx.x * 4;
+        const float* pre = a.hc_pre + (size_t)row * 4;
         const float p0 = pre[0], p1 = pre[1], p2 = pre[2], p3 = pre[3];
         float cv[4][kPer];
 #pragma unroll
@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(kT) k_rowpost(wh_rowpost_args a) {
             xv[k] = acc;
         }
     } else if (a.hc) {
-        const float* pre = a.hc_pre + (size_t)blockIdx.x * a.hc;
+        const float* pre = a.hc_pre + (size_t)row * a.hc;
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
             const uint32_t i = t + kT * k, ic = i < n ? i : 0u;
@@ -229,6 +229,23 @@ __global__ void __launch_bounds__(kT) k_rowpost(wh_rowpost_args a) {
     }
     float* out = a.out + orow * a.ld_out;
     for (uint32_t i = t; i < n; i += kT) out[i] = v[i];
+}
+
+template <int kT>
+__global__ void __launch_bounds__(kT) k_rowpost(wh_rowpost_args a) {
+    wh_rowpost_row<kT>(a, blockIdx.x);
+}
+
+// Two row sets that do not depend on each other in one launch: the low-rank
+// q's norm and the cache rows of a position, each a launch of a few
+// workgroups bound by its chain of barriers (4 to 7 us).
+struct wh_rowpost_pair {
+    wh_rowpost_args r[2];
+};
+template <int kT>
+__global__ void __launch_bounds__(kT) k_rowpost_pair(wh_rowpost_pair p) {
+    const uint32_t first = p.r[0].rows, second = blockIdx.x >= first ? 1u : 0u;
+    wh_rowpost_row<kT>(p.r[second], blockIdx.x - (second ? first : 0u));
 }
 
 // k_rowpost for rows of 512 with the norm (no weights, the sum in the fixed

@@ -3813,6 +3813,21 @@ int rowpost_launch(wh_ctx* c, const wh_rowpost_args& args) {
     return WH_OK;
 }
 
+// Two independent row sets of like size (k_rowpost_pair).
+int rowpost_pair_launch(wh_ctx* c, const wh_rowpost_args& first, const wh_rowpost_args& second) {
+    if (first.rows == 0 || second.rows == 0 || (first.rows < 16) != (second.rows < 16)) {
+        WH_TRY(rowpost_launch(c, first));
+        return rowpost_launch(c, second);
+    }
+    wh_rowpost_pair p{{first, second}};
+    p.r[0].tree = p.r[1].tree = c->exact ? 0u : 1u;
+    const unsigned grid = first.rows + second.rows;
+    if (first.rows < 16) k_rowpost_pair<1024><<<grid, 1024, 0, c->stream>>>(p);
+    else k_rowpost_pair<256><<<grid, 256, 0, c->stream>>>(p);
+    WH_HIP(hipGetLastError());
+    return WH_OK;
+}
+
 wh_rowpost_args rowpost_args(const float* x, float* out, size_t rows, size_t n, size_t ld_in, size_t ld_out) {
     wh_rowpost_args a{};
     a.x = x;
@@ -4072,11 +4087,23 @@ static int mla_decode_impl(wh_ctx* c, const wh_mla_layer* L, size_t token_pos, c
         WH_TRY(launch_fp8(c, *wq_a, 0, q_lora, xq, ql, 1, hidden, q_lora, 0, 0, wkv, 0, head_dim, kvt));
     else
         WH_TRY(launch_fp8(c, *wq_a, 0, q_lora, xq, ql, 1, hidden, q_lora));
+    // kv path (E/compute.rs:4046-4075): wkv, kv norm, RoPE, act-quant of the
+    // non-rope dims, into the cache row of this position, beside the norm and
+    // act-quant of the low-rank q
+    if (!pair) WH_TRY(launch_fp8(c, *wkv, 0, head_dim, xq, kvt, 1, hidden, head_dim));
     a = rowpost_args(ql, ql, 1, q_lora, q_lora, q_lora);
     a.norm = 1;
     a.w = L->q_norm_bf16;
     a.aq_len = (uint32_t)q_lora;
-    WH_TRY(rowpost_launch(c, a));
+    wh_rowpost_args kv = rowpost_args(kvt, kv_row, 1, head_dim, head_dim, head_dim);
+    kv.norm = 1;
+    kv.w = L->kv_norm_bf16;
+    kv.inv_freqs = inv;
+    kv.pairs = (uint32_t)pairs;
+    kv.rope_off = (uint32_t)nope;
+    kv.position = (uint32_t)token_pos;
+    kv.aq_len = (uint32_t)nope;
+    WH_TRY(rowpost_pair_launch(c, a, kv));
     WH_TRY(launch_fp8(c, *wq_b, 0, q_full, ql, q, 1, q_lora, q_full));
     a = rowpost_args(q, q, heads, head_dim, head_dim, head_dim);
     a.norm = 1;
@@ -4084,18 +4111,6 @@ static int mla_decode_impl(wh_ctx* c, const wh_mla_layer* L, size_t token_pos, c
     a.pairs = (uint32_t)pairs;
     a.rope_off = (uint32_t)nope;
     a.position = (uint32_t)token_pos;
-    WH_TRY(rowpost_launch(c, a));
-    // kv path (E/compute.rs:4046-4075): wkv, kv norm, RoPE, act-quant of the
-    // non-rope dims, into the cache row of this position
-    if (!pair) WH_TRY(launch_fp8(c, *wkv, 0, head_dim, xq, kvt, 1, hidden, head_dim));
-    a = rowpost_args(kvt, kv_row, 1, head_dim, head_dim, head_dim);
-    a.norm = 1;
-    a.w = L->kv_norm_bf16;
-    a.inv_freqs = inv;
-    a.pairs = (uint32_t)pairs;
-    a.rope_off = (uint32_t)nope;
-    a.position = (uint32_t)token_pos;
-    a.aq_len = (uint32_t)nope;
     WH_TRY(rowpost_launch(c, a));
     // window softmax with sink (E/compute.rs:4106-4197)
     wh_attn_args w{};
@@ -4208,7 +4223,7 @@ static int mla_decode_batch_impl(wh_ctx* c, const wh_mla_layer* L, const size_t*
     float *xq = base + o_xq, *ql = base + o_ql, *q = base + o_q, *kvt = base + o_kv, *sc = base + o_sc,
           *at = base + o_at, *om = base + o_om;
     // q and kv paths (E/compute.rs:4420-4490): act-quant of every x; wq_a
-    // and wkv over all positions; q norm + act-quant; wq_b over all positions
+    // and wkv over all positions
     wh_rowpost_args a = rowpost_args(in_dev, xq, npos, hidden, in.ld ? in.ld : hidden, hidden);
     a.norm = in.norm ? 1u : 0u;
     a.w = in.w;
@@ -4219,25 +4234,16 @@ static int mla_decode_batch_impl(wh_ctx* c, const wh_mla_layer* L, const size_t*
     WH_TRY(rowpost_launch(c, a));
     WH_TRY(wh_fp8_gemv_multi_pair_async(c, L->wq_a, 0, q_lora, ql, q_lora, L->wkv, 0, head_dim, kvt, head_dim, xq, npos,
                                         hidden));
-    a = rowpost_args(ql, ql, npos, q_lora, q_lora, q_lora);
-    a.norm = 1;
-    a.w = L->q_norm_bf16;
-    a.aq_len = (uint32_t)q_lora;
-    WH_TRY(rowpost_launch(c, a));
-    WH_TRY(wh_fp8_gemv_multi_async(c, L->wq_b, 0, q_full, ql, npos, q_lora, q, q_full));
-    // per position: per-head norm + RoPE of q; kv norm, RoPE, act-quant of
-    // the non-rope dims into the position's cache row; up to WH_POS_BATCH
-    // positions per launch
+    // the low-rank q's norm and act-quant beside the kv norm, RoPE and act-quant
+    // of the non-rope dims into each position's cache row; after wq_b, per
+    // position, the per-head norm + RoPE of q.  Up to WH_POS_BATCH positions
+    // per launch
+    wh_rowpost_args qn = rowpost_args(ql, ql, npos, q_lora, q_lora, q_lora);
+    qn.norm = 1;
+    qn.w = L->q_norm_bf16;
+    qn.aq_len = (uint32_t)q_lora;
     for (size_t c0 = 0; c0 < npos; c0 += WH_POS_BATCH) {
         const size_t nb = std::min<size_t>(WH_POS_BATCH, npos - c0);
-        a = rowpost_args(q + c0 * q_full, q + c0 * q_full, nb * heads, head_dim, head_dim, head_dim);
-        a.norm = 1;
-        a.inv_freqs = inv;
-        a.pairs = (uint32_t)pairs;
-        a.rope_off = (uint32_t)nope;
-        a.rows_per_pos = (uint32_t)heads;
-        for (size_t i = 0; i < nb; ++i) a.bpos[i] = (uint32_t)positions[c0 + i];
-        WH_TRY(rowpost_launch(c, a));
         a = rowpost_args(kvt + c0 * head_dim, kv_cache_dev, nb, head_dim, head_dim, kv_stride);
         a.norm = 1;
         a.w = L->kv_norm_bf16;
@@ -4247,6 +4253,19 @@ static int mla_decode_batch_impl(wh_ctx* c, const wh_mla_layer* L, const size_t*
         a.aq_len = (uint32_t)nope;
         a.rows_per_pos = 1;
         a.out_at_pos = 1;
+        for (size_t i = 0; i < nb; ++i) a.bpos[i] = (uint32_t)positions[c0 + i];
+        if (c0 == 0) WH_TRY(rowpost_pair_launch(c, qn, a));
+        else WH_TRY(rowpost_launch(c, a));
+    }
+    WH_TRY(wh_fp8_gemv_multi_async(c, L->wq_b, 0, q_full, ql, npos, q_lora, q, q_full));
+    for (size_t c0 = 0; c0 < npos; c0 += WH_POS_BATCH) {
+        const size_t nb = std::min<size_t>(WH_POS_BATCH, npos - c0);
+        a = rowpost_args(q + c0 * q_full, q + c0 * q_full, nb * heads, head_dim, head_dim, head_dim);
+        a.norm = 1;
+        a.inv_freqs = inv;
+        a.pairs = (uint32_t)pairs;
+        a.rope_off = (uint32_t)nope;
+        a.rows_per_pos = (uint32_t)heads;
         for (size_t i = 0; i < nb; ++i) a.bpos[i] = (uint32_t)positions[c0 + i];
         WH_TRY(rowpost_launch(c, a));
     }
