@@ -392,6 +392,36 @@ __global__ void __launch_bounds__(256) k_hc_y(wh_hc_args a0) {
     a.y[d] = acc;
 }
 
+// k_hc_post of many streams for hc 4: a thread takes four dims of all four
+// copies, so the residual is read once and in 16-byte pieces instead of once
+// per output copy.  The same terms in the same order.  128 streams, 18.9 MB:
+// 10.4 -> 5.6 us.  Grid (hidden / 1024 rounded up, streams).
+__global__ void __launch_bounds__(256) k_hc_post4(const float* __restrict__ y, const float* __restrict__ res,
+                                                  const float* __restrict__ post, const float* __restrict__ comb,
+                                                  float* __restrict__ out, uint32_t hidden) {
+    const size_t z = blockIdx.y;
+    const uint32_t d4 = blockIdx.x * 256 + threadIdx.x, n4 = hidden / 4;
+    if (d4 >= n4) return;
+    const float4 yv = ((const float4*)y)[z * n4 + d4];
+    float4 rv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rv[i] = ((const float4*)res)[(z * 4 + i) * n4 + d4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float p = post[z * 4 + k];
+        float4 acc = make_float4(p * yv.x, p * yv.y, p * yv.z, p * yv.w);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float c = comb[z * 16 + k * 4 + i];
+            acc.x = acc.x + c * rv[i].x;
+            acc.y = acc.y + c * rv[i].y;
+            acc.z = acc.z + c * rv[i].z;
+            acc.w = acc.w + c * rv[i].w;
+        }
+        ((float4*)out)[(z * 4 + k) * n4 + d4] = acc;
+    }
+}
+
 // hc_post_into: out[k * hidden + d] = post[k] * y[d], then + comb[k][i] *
 // residual[i * hidden + d] for i in order.  Stream z = blockIdx.y of a
 // batched launch: y + z * hidden, residual and out + z * hc * hidden,
