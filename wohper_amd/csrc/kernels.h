@@ -161,19 +161,10 @@ __device__ __forceinline__ void wh_stage_f32_fp8_store(const wh_stage_f32_fp8& s
 }
 
 // ------------------------------------------------------------- act-quant
-// The act-quant of blocks of 64 (E/compute.rs:2504-2521) over n = 64 blocks
-// of values in place: a row of 16 lanes per block, four values a lane, so the
-// values are read and written once in 16-byte pieces and the maximum takes
-// four DPP steps, no LDS and no barrier.  The maximum of a block does not
-// depend on the order (NaN never wins it), so these are the values of
-// k_act_quant_inplace.  Bound by memory: 128 positions x 32768 values, 33.6 MB
-// both ways, 8.5 us against 38.6 us with a workgroup per block (one value in
-// four lanes' loads, two barriers).
-__global__ void __launch_bounds__(256) k_act_quant64_inplace(float* __restrict__ v, uint32_t n) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= n / 4) return;  // whole rows of 16 lanes: n % 64 == 0
-    float4* const p = (float4*)v + i;
-    const float4 x = *p;
+// Act-quant (E/compute.rs:2504-2521) of a block of 64 by a row of 16 lanes,
+// four values each: the block's maximum by four DPP steps (it does not depend
+// on the order, and NaN never wins it).
+__device__ __forceinline__ float4 wh_aq64_quad(float4 x) {
     float amax = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
     amax = fmaxf(amax, wh_dpp_f<0xB1>(amax));
     amax = fmaxf(amax, wh_dpp_f<0x4E>(amax));
@@ -188,7 +179,18 @@ __global__ void __launch_bounds__(256) k_act_quant64_inplace(float* __restrict__
         const float t = e * inv;
         return (t != t ? -480.0f : wh_e4m3_round(wh_clamp448(t))) * scale;
     };
-    *p = make_float4(quant(x.x), quant(x.y), quant(x.z), quant(x.w));
+    return make_float4(quant(x.x), quant(x.y), quant(x.z), quant(x.w));
+}
+
+// n = 64 blocks of values in place, read and written once in 16-byte pieces,
+// no LDS and no barrier: the values of k_act_quant_inplace.  Bound by memory:
+// 128 positions x 32768 values, 33.6 MB both ways, 8.5 us against 38.6 us with
+// a workgroup per block (one value in four lanes' loads, two barriers).
+__global__ void __launch_bounds__(256) k_act_quant64_inplace(float* __restrict__ v, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n / 4) return;  // whole rows of 16 lanes: n % 64 == 0
+    float4* const p = (float4*)v + i;
+    *p = wh_aq64_quad(*p);
 }
 
 // Standalone E/compute.rs:2504-2521 over n values in place, one workgroup per

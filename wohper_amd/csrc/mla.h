@@ -217,7 +217,16 @@ __device__ __forceinline__ void wh_rowpost_row(const wh_rowpost_args& a, uint32_
         }
         __syncthreads();
     }
-    if (a.aq_len) {
+    if (a.aq_len && a.aq_len % 64 == 0) {
+        // whole blocks: 16 lanes each, every thread a quarter of the steps a
+        // value per lane takes (4096 values by 256 threads: the row kernel
+        // 15.8 -> 10.4 us for 128 rows, 13.6 -> 7.1 us for 32)
+        for (uint32_t i = 4 * t; i < a.aq_len; i += 4 * kT) {
+            float4* const p = (float4*)(v + i);
+            *p = wh_aq64_quad(*p);
+        }
+        __syncthreads();
+    } else if (a.aq_len) {
         const uint32_t wave = t >> 6, lane = t & 63;
         for (uint32_t b = wave; b * 64 < a.aq_len; b += kW) {
             const uint32_t i = b * 64 + lane;
