@@ -64,6 +64,24 @@ def test_multi_exact_matches_rows_multi(ctx, oracle, rows, cols, n, r0, r1, ue8m
     ctx.release(t)
 
 
+@pytest.mark.parametrize("rows,cols,n,r0,r1,ue8m0", [
+    (4096, 8192, 2, 0, 4096, False), (4224, 1024, 13, 16, 4209, True), (4224, 2048, 18, 0, 4224, False),
+    (8320, 2048, 9, 0, 8320, True), (8320, 3072, 25, 128, 8320, False), (32768, 1024, 29, 0, 32768, False)])
+def test_multi_exact_matrix_instructions(ctx, oracle, rows, cols, n, r0, r1, ue8m0):
+    """The one-term matrix instructions: one and two row tiles a wave, a partial
+    last row tile, partial tiles of inputs, two and more chunks of columns; an
+    input of tiny values (products and sums below the normal range) and one of
+    large ones keep their own columns."""
+    t, w, scales = _tensor(ctx, rows, cols, rows + cols + n, ue8m0)
+    xs = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    xs[0] *= np.float32(2.0 ** -126)
+    xs[n - 1] *= np.float32(1e30)
+    ys = _run(ctx, t, xs, r0, r1)
+    want = oracle.fp8_gemv_rows_multi(w, rows, cols, scales, rows // 128, cols // 128, xs, r0, r1)
+    assert np.array_equal(bits(ys), bits(np.stack(want)))
+    ctx.release(t)
+
+
 def test_multi_exact_special_codes(ctx, oracle):
     rows, cols, n = 1024, 2048, 16
     t, w, scales = _tensor(ctx, rows, cols, 17, special=True)

@@ -28,6 +28,7 @@
 #include "moe_tok.h"
 #include "fp8_mm.h"
 #include "fp8_tol.h"
+#include "fp8_exact_mm.h"
 #include "fp8_multi.h"
 #include "moe_bmx.h"
 #include "probe.h"
@@ -594,6 +595,39 @@ int launch_fp8(wh_ctx* c, const Tensor& t, size_t r0, size_t r1, const float* x,
             WH_HIP(hipGetLastError());
             return WH_OK;
         }
+    }
+    // several inputs in the reference's order on matrix instructions
+    // (k_fp8_exact_mm).  Its time goes by tiles of 16 inputs, that of the vector
+    // kernel below by inputs, so a tile has to be full enough; one tile against
+    // the vector kernel, us: 4096 x 8192 22.2 (2 to 5 inputs 26, 8 inputs 31, 13
+    // 36), 8192 x 4096 23.6 (5 inputs 18, 8 22, 13 32), 32768 x 1024, where a
+    // workgroup's first loads are most of its time, 27.9 (8 inputs 18, 13 30).
+    // Below 4096 rows the per-input kernel's wider grid is faster.  Two row
+    // tiles a wave where 32-row workgroups still cover the chip's 256 CUs
+    const size_t xrows = (r1 - r0) + (t2 ? r1_2 - r0_2 : 0), tiles = (n_batch + 15) / 16;
+    const size_t tile_min = t.cols <= 1024 ? 13 : xrows > 4096 ? 9 : 2;
+    const auto tile_ok = [](const Tensor& m, size_t row) { return row % 16 == 0 && (m.rows / m.scale_rows) % 16 == 0; };
+    if (n_batch >= 2 && xrows >= 4096 && n_batch >= tile_min * tiles && fp8_split_k(t) && t.cols % (256 * WH_FP8_XMM_GROUPS) == 0 && tile_ok(t, r0) &&
+        (!t2 || (fp8_split_k(*t2) && t2->cols == t.cols && t2->special == t.special &&
+                 t2->scale_fmt == t.scale_fmt && tile_ok(*t2, r0_2))) &&
+        (!x_group_rows || (x_group_rows % 32 == 0 && x_group_stride % 4 == 0)) && x_stride % 4 == 0 &&
+        !((uintptr_t)x & 15) && tiles <= 65535) {
+        const bool pair = xrows / 32 * tiles >= 256;
+        const size_t per = pair ? 32 : 16, b1 = (r1 - r0 + per - 1) / per;
+        if (t2) a.blocks1 = (uint32_t)b1;
+        dim3 grid((unsigned)(b1 + (t2 ? (r1_2 - r0_2 + per - 1) / per : 0)), (unsigned)tiles);
+        const uint32_t n_in = (uint32_t)n_batch;
+        auto go = [&](auto special, auto is_u8) {
+            constexpr bool kSp = decltype(special)::value, kU8 = decltype(is_u8)::value;
+            const size_t lds = per / 16 * (t.cols / 128) * sizeof(float);
+            if (pair) k_fp8_exact_mm<kSp, kU8, 2><<<grid, 256, lds, c->stream>>>(a, n_in);
+            else k_fp8_exact_mm<kSp, kU8, 1><<<grid, 256, lds, c->stream>>>(a, n_in);
+        };
+        using std::bool_constant;
+        if (t.special) u8 ? go(bool_constant<true>(), bool_constant<true>()) : go(bool_constant<true>(), bool_constant<false>());
+        else u8 ? go(bool_constant<false>(), bool_constant<true>()) : go(bool_constant<false>(), bool_constant<false>());
+        WH_HIP(hipGetLastError());
+        return WH_OK;
     }
     // several inputs in the reference's order: each weight byte decoded
     // once for all of them (k_fp8_gemv_multi); the most inputs per
