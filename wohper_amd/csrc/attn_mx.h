@@ -27,13 +27,13 @@ struct wh_attn_f4 {  // four floats at any float's alignment
 } __attribute__((packed, aligned(4)));
 
 // scores[h][j] = exp(q_h . key_j * scale - max of the tile) and tile_max.
-// Grid (ceil(max_keys / 32), ceil(heads / (16 kH)), positions), 256 threads:
-// wave w adds a quarter of the dims for 16 kH heads x 32 keys straight from
-// global memory (a lane's 16 bytes are four dims of its row, the same four on
-// both sides), LDS only joins the quarters.  16 heads a workgroup leave one
-// position enough workgroups; 32 read a key half as often.
-template <int kH>
+// Grid (ceil(max_keys / 32), ceil(heads / 16), positions), 256 threads: wave w
+// adds a quarter of the dims for 16 heads x 32 keys straight from global
+// memory (a lane's 16 bytes are four dims of its row, the same four on both
+// sides), LDS only joins the quarters.  For few positions, which 16 heads a
+// workgroup leave enough workgroups; a batch takes k_attn_scores_mx_tile.
 __global__ void __launch_bounds__(256) k_attn_scores_mx(wh_attn_args a) {
+    constexpr int kH = 1;  // 16-head tiles
     constexpr int kS = 4;  // 16-dim steps requested together
     constexpr int kE = 2 * kH, kLanes = 32 / kE;
     __shared__ __align__(16) float red[4][2 * kH][256];
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256) k_attn_scores_mx(wh_attn_args a) {
 // step of a tile).  Read straight into the operands, every lane's 16 bytes
 // were a row of their own, 64 cache lines an instruction, and a quarter of
 // the dims a wave shared nothing.  64 heads x 628 keys of 32 positions:
-// 40.5 -> 25.2 us (8.4 us of matrix time at 157 TFLOP/s).  The row stride of
+// 40.5 -> 25.8 us (8.4 us of matrix time at 157 TFLOP/s).  The row stride of
 // 68 floats puts the 16 rows of a read on 16 bank groups.
 __global__ void __launch_bounds__(256) k_attn_scores_mx_tile(wh_attn_args a) {
     constexpr uint32_t kLd = 68;
@@ -179,9 +179,7 @@ __global__ void __launch_bounds__(256) k_attn_scores_mx_tile(wh_attn_args a) {
     __syncthreads();
     auto step = [&](uint32_t k, int b) {
         request(b, k + 2);
-        __builtin_amdgcn_sched_barrier(0);
         multiply(b);
-        __builtin_amdgcn_sched_barrier(0);
         store(b ^ 1);
         __syncthreads();
     };

@@ -3878,7 +3878,7 @@ void attn_mx_launch(wh_ctx* c, const wh_attn_args& a, unsigned nb) {
     const unsigned g16 = (a.heads + 15) / 16, g32 = (a.heads + 31) / 32;
     const unsigned wide = (a.max_keys + 63) / 64;
     if ((size_t)wide * g32 * nb >= 256) k_attn_scores_mx_tile<<<dim3(wide, g32, nb), 256, 0, c->stream>>>(a);
-    else k_attn_scores_mx<1><<<dim3(tiles, g16, nb), 256, 0, c->stream>>>(a);
+    else k_attn_scores_mx<<<dim3(tiles, g16, nb), 256, 0, c->stream>>>(a);
     if ((size_t)(a.head_dim / 64) * g32 * nb >= 256)
         k_attn_weighted_mx<2, 4><<<dim3(a.head_dim / 64, g32, nb), 256, 0, c->stream>>>(a);
     else k_attn_weighted_mx<1, 1><<<dim3(a.head_dim / 16, g16, nb), 256, 0, c->stream>>>(a);
