@@ -228,51 +228,38 @@ __global__ void __launch_bounds__(256) k_attn_weighted_mx(wh_attn_args a) {
     __shared__ float den_s[4][16 * kH], max_s[16 * kH];
     __shared__ float f_s[16 * kH][WH_ATTN_MX_TILES + 1];  // exp(tile max - max)
     const wh_attn_pos v = wh_attn_resolve(a, blockIdx.z);
-    const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63, col = lane & 15, q = lane >> 4;
+    const uint32_t t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, col = lane & 15, q = lane >> 4;
     const uint32_t nk = v.n_win + v.n_comp, hd = a.head_dim;
     const uint32_t d0 = blockIdx.x * (16 * kD), h0 = blockIdx.y * (16 * kH);
-    const uint32_t nt = (nk + WH_ATTN_MX_KEYS - 1) / WH_ATTN_MX_KEYS, units = (nk + 15) / 16;
+    const uint32_t nt = (nk + WH_ATTN_MX_KEYS - 1) / WH_ATTN_MX_KEYS, n_full = nk / 16;
     const float* wrow[kH];
 #pragma unroll
     for (int h = 0; h < kH; ++h) wrow[h] = v.scores + (size_t)min(h0 + 16 * h + col, a.heads - 1) * nk;
     float w[2][kH][4], x[2][4][kD];
-    // 16 keys from 16 u: lane q the keys 4 q .. + 3 of its head and of its dims;
-    // past the last key nothing is read and both are 0
+    // 16 keys from 16 u: lane q the keys 4 q .. + 3 of its head and of its dims.
+    // Whole units only, always as many loads and no branch, so that two units
+    // stay in flight (with a branch for a partial one every product waited for
+    // every load: one position over 1128 keys 18.3 us then, 16.0 us so, both
+    // launches); a last partial unit comes after the loop
     auto request = [&](int b, uint32_t u) {
-        const uint32_t j = 16 * u + 4 * q;
-        if (16 * u + 16 <= nk) {  // uniform
+        const uint32_t j = 16 * min(u, n_full - 1) + 4 * q;
 #pragma unroll
-            for (int h = 0; h < kH; ++h) {
-                const wh_attn_f4 p = *(const wh_attn_f4*)(wrow[h] + j);
+        for (int h = 0; h < kH; ++h) {
+            const wh_attn_f4 p = *(const wh_attn_f4*)(wrow[h] + j);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) w[b][h][i] = p.v[i];
-            }
+            for (int i = 0; i < 4; ++i) w[b][h][i] = p.v[i];
+        }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float* row = wh_attn_key(a, v, j + i) + d0 + col;
+        for (int i = 0; i < 4; ++i) {
+            const float* row = wh_attn_key(a, v, j + i) + d0 + col;
 #pragma unroll
-                for (int c = 0; c < kD; ++c) x[b][i][c] = row[16 * c];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool on = j + i < nk;
-                const uint32_t jc = on ? j + i : nk - 1;
-                const float* row = wh_attn_key(a, v, jc) + d0 + col;
-#pragma unroll
-                for (int c = 0; c < kD; ++c) {
-                    const float xv = row[16 * c];
-                    x[b][i][c] = on ? xv : 0.0f;
-                }
-#pragma unroll
-                for (int h = 0; h < kH; ++h) {
-                    const float wv = wrow[h][jc];
-                    w[b][h][i] = on ? wv : 0.0f;
-                }
-            }
+            for (int c = 0; c < kD; ++c) x[b][i][c] = row[16 * c];
         }
     };
-    if (wave < units) request(0, wave);
+    if (n_full) {  // uniform
+        request(0, wave);
+        request(1, wave + 4);
+    }
     // the heads' maxima and their tiles' factors: 16 threads a head
 #pragma unroll
     for (int h = 0; h < kH; ++h) {
@@ -316,12 +303,31 @@ __global__ void __launch_bounds__(256) k_attn_weighted_mx(wh_attn_args a) {
             }
         }
     };
-    for (uint32_t u = wave; u < units; u += 8) {
-        if (u + 4 < units) request(1, u + 4);
+    for (uint32_t u = wave; u < n_full; u += 8) {
         multiply(0, u);
-        if (u + 4 >= units) break;
-        if (u + 8 < units) request(0, u + 8);
-        multiply(1, u + 4);
+        request(0, u + 8);
+        if (u + 4 < n_full) multiply(1, u + 4);  // uniform, and no loads in it
+        request(1, u + 12);
+    }
+    if (nk % 16 && wave == (n_full & 3)) {  // uniform: the wave with the fewest units
+        const uint32_t j = 16 * n_full + 4 * q;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool on = j + i < nk;
+            const uint32_t jc = on ? j + i : nk - 1;
+            const float* row = wh_attn_key(a, v, jc) + d0 + col;
+#pragma unroll
+            for (int c = 0; c < kD; ++c) {
+                const float xv = row[16 * c];
+                x[0][i][c] = on ? xv : 0.0f;
+            }
+#pragma unroll
+            for (int h = 0; h < kH; ++h) {
+                const float wv = wrow[h][jc];
+                w[0][h][i] = on ? wv : 0.0f;
+            }
+        }
+        multiply(0, n_full);
     }
 #pragma unroll
     for (int h = 0; h < kH; ++h) {
