@@ -24,9 +24,7 @@
 #pragma once
 #include "moe_px.h"
 
-#ifndef WH_BMX_DEPTH
-#define WH_BMX_DEPTH 5  // weight blocks of a wave in flight
-#endif
+#define WH_BMX_DEPTH 4  // weight blocks of a wave in flight (even, and dividing an item's blocks)
 #define WH_BMX_TOK 16u                             // slots per virtual expert
 
 // LDS of one staged virtual expert over `cols` input columns: 16 code
@@ -52,20 +50,13 @@ __device__ __forceinline__ const uint8_t* wh_uni(const uint8_t* p) {
 // types: through HIP's struct uint4 the address space is lost again).
 #define WH_GLOBAL __attribute__((address_space(1)))
 typedef unsigned int wh_u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int wh_u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint4 wh_ld16_global(const void* p) {
     const wh_u32x4 v = *(const WH_GLOBAL wh_u32x4*)p;
     return make_uint4(v.x, v.y, v.z, v.w);
 }
-__device__ __forceinline__ uint2 wh_ld8_global(const void* p) {
-    const wh_u32x2 v = *(const WH_GLOBAL wh_u32x2*)p;
-    return make_uint2(v.x, v.y);
-}
-__device__ __forceinline__ void wh_mx_raw_load_global(wh_mx_raw& r, const uint8_t* wlane, const uint8_t* srow,
-                                                      uint32_t blk) {
+__device__ __forceinline__ void wh_mx_raw_load_global(wh_mx_raw& r, const uint8_t* wlane, uint32_t blk) {
     r.p = wh_ld16_global(wlane + blk * 128);
     r.q = wh_ld16_global(wlane + blk * 128 + 16);
-    r.s = wh_ld8_global(srow + blk * 8);
 }
 
 // Gate/up of the MFMA experts in fp32, for a batch with an inf or NaN input
@@ -115,7 +106,7 @@ __global__ void __launch_bounds__(512, 1) k_moe_batch_mx(wh_batch_args a) {
     constexpr uint32_t CPS = kCols / 16;  // 16-byte pieces of a code record
     constexpr int D = WH_BMX_DEPTH;
     static_assert(NB == 8 || NB == 16, "2048 or 4096 columns");
-    static_assert(D < (int)NB, "the ring spans at most two items");
+    static_assert(D < (int)NB && NB % D == 0 && D % 2 == 0, "block b in ring slot b % D, at most two items in the ring");
     // timeline points (builds with -DWH_TIMELINE): 0 start, 1 ring issued,
     // 2 B staged, 3 the wave's last item done, 4 the workgroup's end
     WH_TL(kGate ? 0 : 1, 0);
@@ -168,13 +159,17 @@ __global__ void __launch_bounds__(512, 1) k_moe_batch_mx(wh_batch_args a) {
     const uint32_t m = kGate ? (rel_##q - q * per_v) & 1 : 0
         // issue side of the ring: block iss_blk of item iss_it; past the
         // wave's last item every step repeats the last block issued (its
-        // result is not used), so each step issues the same three loads and
-        // the waits stay vmcnt(3 (D - 1)) rather than vmcnt(0)
+        // result is not used), so each turn of the ring issues the same loads
+        // and the waits count them rather than wait for all.  A row's scales
+        // come for two blocks at a time, with the odd one: they are a third of
+        // the loads otherwise (read alone with the weights, 5.64 TB/s against
+        // 6.06 without them), and 16 bytes cost what 8 do: 64
+        // tokens' gate/up 265 -> 238 us, 128 tokens' 446 -> 414 us
         uint32_t iss_it = wh_uni(ps + wave), iss_blk = 0, nxt_it = iss_it;
         const uint8_t* iw = w0a;
         const uint8_t* is = s0a;
         uint32_t ib = 0;
-#define WH_BMX_ISSUE(rg, dep)                                                                            \
+#define WH_BMX_ISSUE(d, dep)                                                                             \
     do {                                                                                                 \
         if (iss_it < pe) {                                                                               \
             WH_BMX_ITEM(iss_it, iq, itile, im);                                                          \
@@ -189,12 +184,14 @@ __global__ void __launch_bounds__(512, 1) k_moe_batch_mx(wh_batch_args a) {
                 iss_it = nxt_it = wh_uni((uint32_t)__shfl(nx, 0, 64));                                   \
             }                                                                                            \
         }                                                                                                \
-        wh_mx_raw_load_global(rg, iw + (dep), is + (dep), ib);                                           \
+        wh_mx_raw_load_global(ring[d], iw + (dep), ib);                                                  \
+        if ((d) & 1) rs[(d) / 2] = wh_ld16_global(is + (dep) + (ib & ~1u) * 8);                          \
     } while (0)
         wh_mx_raw ring[D];
+        uint4 rs[D / 2];  // scales of the blocks in slots 2 k, 2 k + 1
         if (iss_it < pe) {
 #pragma unroll
-            for (int d = 0; d < D; ++d) WH_BMX_ISSUE(ring[d], 0u);
+            for (int d = 0; d < D; ++d) WH_BMX_ISSUE(d, 0u);
         }
         __builtin_amdgcn_sched_barrier(0);
         WH_TL(kGate ? 0 : 1, 1);
@@ -250,8 +247,9 @@ __global__ void __launch_bounds__(512, 1) k_moe_batch_mx(wh_batch_args a) {
                 wh_mx_bop bo;
                 wh_mx_bop_load(bo, buf + nl * TS + 256 * cur_blk + dep,
                                buf + WH_BMX_TOK * TS + nl * G + 8 * cur_blk + dep, g);
+                ring[d].s = d & 1 ? make_uint2(rs[d / 2].z, rs[d / 2].w) : make_uint2(rs[d / 2].x, rs[d / 2].y);
                 wh_px_step(acc, ring[d], dep, bo, g);
-                WH_BMX_ISSUE(ring[d], dep);
+                WH_BMX_ISSUE(d, dep);
                 if (++cur_blk == NB) {
                     // C[4 (L / 16) + r][L % 16]: rows of the tile, slot nl
                     asm volatile("" : "+v"(acc));
