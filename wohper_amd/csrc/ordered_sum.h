@@ -21,9 +21,17 @@
 //              by induction every x is the sequential sum.  If not, the runs
 //              just made replace their entries in the tables, and steps 3 and
 //              4 are done again: the chunks up to the first wrong one are
-//              right from then on, so at most C rounds are made, whatever the
-//              values (infinities and NaN too; C rounds are as many adds as
-//              the plain sum has).
+//              right from then on, whatever the values (infinities and NaN
+//              too);
+//   5. plain   where more than a quarter of the chunks left are wrong, the
+//              terms from that group on are added one by one instead.
+//
+// A round fixes one wrong chunk or more and takes 2.0 us (16384 terms), the
+// plain adds of a chunk 0.9 us.  Rows whose neighbouring products cancel to
+// 1e-2 or closer would take nearly a round a chunk (their roundings follow the
+// terms' grid, not the sum's, so starts 8 ulps apart do not go the same way):
+// hc_pre of 4 x 4096 such products 141 us, 68 with step 5, 66 when one lane
+// added every row and 22 on N(0, 1) products (2 chunks wrong at first).
 //
 // On N(0, 1) products 16384 terms take 1.7 rounds on average (the walk meets
 // a power of two inside a chunk, where the rounding grid changes), a sum of
@@ -80,12 +88,42 @@ struct wh_osum_lds {
     float sums[kC];
 };
 
+// acc + the terms from chunk c on, one after the other, by one wave: 32 terms
+// at a time from two register sets.
+template <int kL, int kC>
+__device__ __forceinline__ float wh_osum_plain(const wh_osum_lds<kL, kC>& s, int c, float acc) {
+    constexpr int kB = kL * kC / 32;
+    float4 p[2][8];
+    auto rd = [&](int set, int b) {
+        const float* src = s.rows + wh_osum_at<kL>(32 * b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[set][i] = *(const float4*)(src + 4 * i);
+    };
+    auto add = [&](int set) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = (((acc + p[set][i].x) + p[set][i].y) + p[set][i].z) + p[set][i].w;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int b = c * (kL / 32);
+    rd(0, b);
+#pragma unroll 1
+    for (; b + 1 < kB; b += 2) {
+        rd(1, b + 1);
+        add(0);
+        rd(0, b + 2 < kB ? b + 2 : 0);
+        add(1);
+    }
+    if (b < kB) add(0);
+    return acc;
+}
+
 // acc0 + term 0 + ... in order, for a workgroup of kT >= 256 threads (all of
 // them call; the rows' stores need no barrier before).  kC is 32 or 64.  The
 // result is valid in wave 0.
 template <int kT, int kL, int kC>
 __device__ __forceinline__ float wh_ordered_sum_wg(wh_osum_lds<kL, kC>& s, float acc0) {
-    static_assert(kT >= 256 && (kC == 32 || kC == 64) && kL >= 16 && kL % 16 == 0, "");
+    static_assert(kT >= 256 && (kC == 32 || kC == 64) && kL % 32 == 0, "");
     const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
     // 1. unordered chunk sums: kP threads per chunk
     constexpr int kP0 = kT / kC < 16 ? kT / kC : 16, kP = kP0 < kL / 4 ? kP0 : kL / 4;
@@ -161,6 +199,8 @@ __device__ __forceinline__ float wh_ordered_sum_wg(wh_osum_lds<kL, kC>& s, float
         // the chunks up to the first wrong one start right: go on from its group
         from = __builtin_ctzll(wrong) / 8;
         x_from = __builtin_amdgcn_readlane(xc, 8 * from);
+        if (4 * __builtin_popcountll(wrong) > kC - 8 * from)
+            return wh_osum_plain(s, 8 * from, __int_as_float(x_from));
         if (lane < kC) {
             s.h[c * 8 + (xc & 7)] = __int_as_float(xc);
             s.e[c * 8 + (xc & 7)] = a[0];
