@@ -61,6 +61,29 @@ __device__ __forceinline__ float wh_hc_wave_sum(float v) {
     return v;
 }
 
+// Ordered sums of short rows: workgroup c runs chain c as below, one lane
+// adding the products.  hc_pre of 4 x 64 terms 9.5 us (with k_hc_chains 12),
+// 4 x 256 12.1 (12.9), 1 x 1024 14.9 (15.6); 4 x 512 16.1 against 14.0 there.
+#define WH_HC_LANE_TERMS 1280u
+__global__ void __launch_bounds__(256) k_hc_chains_lane(wh_hc_args a0) {
+    const wh_hc_args a = wh_hc_at(a0, blockIdx.z);
+    __shared__ __align__(16) float prod[WH_HC_LANE_TERMS];
+    const uint32_t t = threadIdx.x, c = blockIdx.x;
+    const float* row = c < a.mix_hc ? a.fn + (size_t)c * a.hc_dim : a.x;
+    constexpr uint32_t kPer = WH_HC_LANE_TERMS / 256;
+    float w[kPer], xv[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t i = t + 256 * k, ic = i < a.hc_dim ? i : 0u;
+        xv[k] = a.x[ic];
+        w[k] = row[ic];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) prod[t + 256 * k] = w[k] * xv[k];
+    __syncthreads();
+    if (t == 0) a.sums[c] = wh_ordered_sum_lds(prod, a.hc_dim, 0.0f);
+}
+
 // Ordered sums: workgroup c (1024 threads) runs chain c < mix_hc (fn row
 // c . x) or, for c = mix_hc, the sum of squares, each product rounded on its
 // own and added in order (ordered_sum.h), segments of kL * kC terms at a time

@@ -4418,16 +4418,17 @@ int hc_pre_launch(wh_ctx* c, const float* fn_dev, const float* scale_dev, const 
     a.pre = a.sums + npos * a.sums_ld;
     const unsigned z = (unsigned)npos;
     if (c->exact) {
-        // the smallest chunks that hold the row (C = 32 chunks up to 4096
-        // terms, 64 above: the chain over the chunks costs about 45 cycles a
-        // chunk, the two runs over a chunk 9 cycles a term each); rows past
-        // 16384 terms go on in segments of that
+        // short rows one lane each; else the smallest chunks that hold the row
+        // (C = 32 chunks up to 4096 terms, 64 above: the chain over the chunks
+        // costs about 45 cycles a chunk, the two runs over a chunk 9 cycles a
+        // term each); rows past 16384 terms go on in segments of that
         auto chains = [&](auto l, auto n) {
             constexpr int kL = decltype(l)::value, kC = decltype(n)::value;
             k_hc_chains<kL, kC><<<dim3(a.mix_hc + 1, 1, z), 1024, sizeof(wh_osum_lds<kL, kC>), c->stream>>>(a);
         };
         using std::integral_constant;
-        if (a.hc_dim <= 1024) chains(integral_constant<int, 32>(), integral_constant<int, 32>());
+        if (a.hc_dim <= WH_HC_LANE_TERMS) k_hc_chains_lane<<<dim3(a.mix_hc + 1, 1, z), 256, 0, c->stream>>>(a);
+        else if (a.hc_dim <= 2048) chains(integral_constant<int, 64>(), integral_constant<int, 32>());
         else if (a.hc_dim <= 4096) chains(integral_constant<int, 128>(), integral_constant<int, 32>());
         else if (a.hc_dim <= 8192) chains(integral_constant<int, 128>(), integral_constant<int, 64>());
         else chains(integral_constant<int, 256>(), integral_constant<int, 64>());
