@@ -241,3 +241,31 @@ def test_hc_pre_short_rows_time(ctx, dev):
             ctx.set_exact_numerics(True)
     print(f"hc_pre 4 x 64: exact {us[True]:.1f} us, order-free {us[False]:.1f} us")
     assert us[True] <= 1.15 * us[False]
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties", "range"])
+@pytest.mark.parametrize("n", [575, 576, 577, 1500, 2047, 2048, 2049])
+@pytest.mark.parametrize("rows", [3, 17])
+def test_rms_norm_ordered_sum_edges(ctx, oracle, dev, kind, n, rows):
+    """The last row that one lane adds and the chunk sizes after it, bit for
+    bit."""
+    test_rms_norm_ordered_sum(ctx, oracle, dev, kind, n, rows)
+
+
+def test_rms_norm_one_wave_more_than_512(ctx, dev):
+    """One row of 513 terms, one more than a row of 512 whose adds one lane
+    makes: as long as that (4.0 us each; through the chunked sum 4.6)."""
+    us = {}
+    ctx.set_exact_numerics(True)
+    for n in (512, 513):
+        x, o = dev.put(np.random.default_rng(n).standard_normal(n).astype(np.float32)), dev.empty(4 * n)
+        g = ctx.graph_capture(lambda: [ctx.rms_norm_async(x, o, 1, n) for _ in range(50)])
+        t = []
+        for _ in range(8):
+            ctx.timer_start()
+            ctx.graph_launch(g)
+            t.append(ctx.timer_stop() / 50)
+        ctx.graph_release(g)
+        us[n] = min(t)
+    print(f"norm of one row: 512 {us[512]:.2f} us, 513 {us[513]:.2f} us")
+    assert us[513] <= 1.08 * us[512]

@@ -138,11 +138,12 @@ __device__ __forceinline__ void wh_rowpost_row(const wh_rowpost_args& a, uint32_
         if (i >= n) xv[k] = 0.0f;
         wv[k] = use_w && i < n ? wh_bf16_value((uint16_t)wr[k]) : 1.0f;
     }
+    if (!a.norm) {
 #pragma unroll
-    for (int k = 0; k < kPer; ++k)
-        if (t + kT * k < n) v[t + kT * k] = xv[k];
-    __syncthreads();
-    if (a.norm) {
+        for (int k = 0; k < kPer; ++k)
+            if (t + kT * k < n) v[t + kT * k] = xv[k];
+        __syncthreads();
+    } else {
         if (a.tree) {
             // each thread its strided terms, then the wave butterfly, then
             // the waves in order: the same value up to rounding
@@ -162,8 +163,8 @@ __device__ __forceinline__ void wh_rowpost_row(const wh_rowpost_args& a, uint32_
         } else {
             // the reference's order: every product rounded on its own, then
             // the sequential sum by the whole workgroup (ordered_sum.h); up
-            // to 512 terms one lane adds them: 64 heads of 512 took 7.3 us
-            // that way and 8.6 us with the tables and the check
+            // to 576 terms one lane adds them (one row of 513 4.0 us that
+            // way and 4.6 with the tables and the check, of 600 5.1 and 4.6)
             constexpr int kMaxL = WH_ROWPOST_MAX / 32;
             __shared__ __align__(16) wh_osum_lds<kMaxL, 32> os;
             auto stage = [&](auto l) {
@@ -177,14 +178,16 @@ __device__ __forceinline__ void wh_rowpost_row(const wh_rowpost_args& a, uint32_
                 return wh_ordered_sum_wg<kT, kL, 32>(s, 0.0f);
             };
             float s;
-            if (n <= 512) {
+            if (n <= 576) {
 #pragma unroll
-                for (int k = 0; k < 512 / kT + (kT > 512); ++k)
+                for (int k = 0; k < (576 + kT - 1) / kT; ++k)
                     if (t + kT * k < n) os.rows[t + kT * k] = xv[k] * xv[k];
                 __syncthreads();
                 s = t == 0 ? wh_ordered_sum_lds(os.rows, n, 0.0f) : 0.0f;
             } else if (n <= 1024) {
                 s = stage(std::integral_constant<int, 32>());
+            } else if (n <= 2048) {
+                s = stage(std::integral_constant<int, 64>());
             } else {
                 s = stage(std::integral_constant<int, kMaxL>());
             }
