@@ -484,8 +484,8 @@ int wh_fp8_gemv_multi_async(wh_ctx* ctx, wh_tensor w, size_t row_start, size_t r
  * [row_start0, row_end0) of w0 into y0_dev and rows [row_start1, row_end1) of
  * w1 into y1_dev (wq_a and wkv of a batch of decode positions; the reference
  * calls rows_multi once for each, E/compute.rs:4005-4013, 6384-6577).
- * Results are those of the two calls; when both take the MFMA path (for up to
- * 16 inputs or under 256 rows: with the same k split), the tensors share width, scale format, rows per scale row and
+ * Results are those of the two calls; when both take the MFMA path with the
+ * same k split, the tensors share width, scale format, rows per scale row and
  * the special-code flag, and neither output overlaps the inputs or the other
  * output, they go out as one launch. */
 int wh_fp8_gemv_multi_pair_async(wh_ctx* ctx, wh_tensor w0, size_t row_start0, size_t row_end0, float* y0_dev,

@@ -306,3 +306,64 @@ def test_fp8_mfma_wide_pair_and_groups(ctx, n):
         ctx.release(t)
     ctx.device_free(xd)
     ctx.device_free(yd)
+
+
+def _graph_us(ctx, fn, reps=20):
+    """Time of one fn(), `reps` of them in a graph."""
+    fn()
+    ctx.synchronize()
+    g = ctx.graph_capture(lambda: [fn() for _ in range(reps)])
+    us = []
+    for _ in range(6):
+        ctx.timer_start()
+        ctx.graph_launch(g)
+        us.append(ctx.timer_stop() / reps)
+    ctx.graph_release(g)
+    return min(us)
+
+
+@pytest.mark.parametrize("rows,cols,n", [((8192, 512), 1024, 64), ((4096, 1024), 4096, 32), ((1024, 512), 4096, 128)])
+def test_pair_of_two_k_splits_time(ctx, rows, cols, n):
+    """Two tensors that take different k splits are not slower as a pair than
+    as two calls (in one launch, whose workgroups of the first last as long as
+    the launch, 1.2 to 1.5 times their time)."""
+    ts = [ctx.store_fp8_synthetic(r, cols, 3, r, np.full((r // 128, cols // 128), 2.0 ** -10, np.float32)) for r in rows]
+    x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    xd, y = ctx.device_alloc(x.nbytes), [ctx.device_alloc(4 * n * r) for r in rows]
+    ctx.to_device(xd, x)
+    pair = _graph_us(ctx, lambda: ctx.fp8_gemv_multi_pair_async(ts[0], 0, rows[0], y[0], rows[0], ts[1], 0, rows[1], y[1],
+                                                                rows[1], xd, n, cols))
+    two = _graph_us(ctx, lambda: [ctx.fp8_gemv_multi_async(t, 0, r, xd, n, cols, p, r) for t, r, p in zip(ts, rows, y)])
+    print(f"{rows} x {cols}, {n} inputs: pair {pair:.1f} us, two calls {two:.1f} us")
+    for t in ts:
+        ctx.release(t)
+    for p in (xd, *y):
+        ctx.device_free(p)
+    assert pair <= 1.1 * two
+
+
+def test_pair_past_one_grid(ctx):
+    """A pair whose row blocks pass a grid of 65535 with the second tensor's k
+    split, but not with each tensor's own: it runs, as two calls."""
+    rows, cols, n = (128 * 16384, 256), 1024, 17
+    ts = [ctx.store_fp8_synthetic(r, cols, 3, r, np.full((r // 128, cols // 128), 2.0 ** -10, np.float32)) for r in rows]
+    x = np.random.default_rng(2).standard_normal((n, cols)).astype(np.float32)
+    xd, y = ctx.device_alloc(x.nbytes), [ctx.device_alloc(4 * n * r) for r in rows]
+    ctx.to_device(xd, x)
+    got = []
+    for pair in (True, False):
+        if pair:
+            ctx.fp8_gemv_multi_pair_async(ts[0], 0, rows[0], y[0], rows[0], ts[1], 0, rows[1], y[1], rows[1], xd, n, cols)
+        else:
+            for t, r, p in zip(ts, rows, y):
+                ctx.fp8_gemv_multi_async(t, 0, r, xd, n, cols, p, r)
+        out = [np.empty((n, r), np.float32) for r in rows]
+        for o, p in zip(out, y):
+            ctx.from_device(o, p)
+        got.append(out)
+    for t in ts:
+        ctx.release(t)
+    for p in (xd, *y):
+        ctx.device_free(p)
+    for a, b in zip(*got):
+        assert np.any(a) and np.array_equal(a.view(np.uint32), b.view(np.uint32))

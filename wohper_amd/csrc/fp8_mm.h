@@ -71,9 +71,6 @@ struct wh_fp8mm_args {
     const void* scales2;
     float* y2;
     uint32_t row_start2, row_end2, y2_stride, rb_first;
-    // k_fp8_mm_wide only: the second tensor's k split, which may be another,
-    // and the splits between two blocks' partial tiles (the larger count)
-    uint32_t kc2, splits2, ws_splits;
 };
 
 // Two f32 to two bf16, each rounded to nearest even (v_cvt_pk_bf16_f32).
@@ -311,7 +308,7 @@ __global__ void __launch_bounds__(512, WH_FP8MM_WG_PER_CU) k_fp8_mm(wh_fp8mm_arg
 // staging stores of 16 lanes contiguous.
 #define WH_FP8MMW_ROWS 256u  // rows per workgroup: 4 waves x 64
 
-// grid (row blocks, most splits of a tensor, blocks of 16 kT inputs), 256 threads
+// grid (row blocks, k splits, blocks of 16 kT inputs), 256 threads
 template <bool kSpecial, bool kScaleU8, int kT>
 __global__ void __launch_bounds__(256, 2) k_fp8_mm_wide(wh_fp8mm_args a) {
     static_assert(kT >= 2 && kT <= 4, "a stage is at most 64 inputs x groups");
@@ -324,8 +321,6 @@ __global__ void __launch_bounds__(256, 2) k_fp8_mm_wide(wh_fp8mm_args a) {
     const uint32_t rb = blockIdx.x, ks = blockIdx.y, tb = blockIdx.z;
     const uint32_t wave = threadIdx.x >> 6, L = threadIdx.x & 63, q = L >> 4, col = L & 15;
     const bool t2 = rb >= a.rb_first;
-    const uint32_t splits = t2 ? a.splits2 : a.splits;
-    if (ks >= splits) return;
     const uint8_t* const W = t2 ? a.w2 : a.w;
     const void* const SC = t2 ? a.scales2 : a.scales;
     float* const Y = t2 ? a.y2 : a.y;
@@ -334,7 +329,7 @@ __global__ void __launch_bounds__(256, 2) k_fp8_mm_wide(wh_fp8mm_args a) {
     const uint32_t rbl = t2 ? rb - a.rb_first : rb;
     const uint32_t r0 = row_start + rbl * kRows + 16 * kR * wave;  // the wave's first row
     const uint32_t grp = a.xg_shift < 31 ? (rbl * kRows) >> a.xg_shift : 0;
-    const uint32_t G = (t2 ? a.kc2 : a.kc) >> 7, g0 = ks * G;
+    const uint32_t G = a.kc >> 7, g0 = ks * G;
     // staging: thread (group, input tile | h, half | input of the tile); inputs
     // past the end stage the last one's values, whose sums are not stored
     const uint32_t sgs = kT == 2 ? wave >> 1 : 0, stt = kT == 2 ? wave & 1 : wave;
@@ -433,11 +428,11 @@ __global__ void __launch_bounds__(256, 2) k_fp8_mm_wide(wh_fp8mm_args a) {
         }
     }
     // D[4 q + r][col]: input 4 q + r of the tile, row `col` of the tile
-    if (splits > 1) {
+    if (a.splits > 1) {
         // partial tiles in register order; the last workgroup of the block sums
         // the splits in order
         constexpr uint32_t kTile = kRows * kTok;
-        const size_t tile = ((size_t)tb * a.row_blocks + rb) * a.ws_splits;
+        const size_t tile = ((size_t)tb * a.row_blocks + rb) * a.splits;
         float* const wsp = a.ws + (tile + ks) * kTile + (size_t)wave * (kTile / 4) + L;
 #pragma unroll
         for (int i = 0; i < kR; ++i)
@@ -450,13 +445,13 @@ __global__ void __launch_bounds__(256, 2) k_fp8_mm_wide(wh_fp8mm_args a) {
         uint32_t* const last = (uint32_t*)xs;
         if (threadIdx.x == 0) {
             uint32_t* cnt = a.cnt + (size_t)tb * a.row_blocks + rb;
-            *last = wh_arrive(cnt) + 1 == splits;
+            *last = wh_arrive(cnt) + 1 == a.splits;
             if (*last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
         if (!*last) return;
         const float* const wt = a.ws + tile * kTile + (size_t)wave * (kTile / 4) + L;
-        for (uint32_t sp = 0; sp < splits; ++sp) {
+        for (uint32_t sp = 0; sp < a.splits; ++sp) {
 #pragma unroll
             for (int i = 0; i < kR; ++i)
 #pragma unroll

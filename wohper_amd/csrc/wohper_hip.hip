@@ -752,10 +752,9 @@ struct Fp8MmSecond {
 };
 
 // The launch of a multi-input MFMA product: kt = 0 for k_fp8_mm, else
-// k_fp8_mm_wide with 16 kt inputs per workgroup; kg (kg2: of the second
-// tensor) groups per k split.
+// k_fp8_mm_wide with 16 kt inputs per workgroup; kg groups per k split.
 struct Fp8MmPlan {
-    size_t kg = 0, kg2 = 0;
+    size_t kg = 0;
     int kt = 0;
 };
 
@@ -766,28 +765,24 @@ struct Fp8MmPlan {
 //    counted in units of 256 rows x 32 inputs x 128 columns, is at most 1024:
 //    1024 x 4096 takes 10 us there for 64 inputs and 12 for 128 (wide: 14 to 18);
 //    32768 x 1024 and 4096 x 8192 the same in both for 32; at the next step, 40
-//    inputs, they take 22.6 and 29.8 us there and 20.6 and 25.0 us wide;
-//  - two tensors whose k splits differ (k_fp8_mm needs one launch for each):
-//    wide, 1024 + 512 rows x 4096 for 192 inputs 33 -> 19 us.
+//    inputs, they take 22.6 and 29.8 us there and 20.6 and 25.0 us wide.
+// With rows2 more of a second tensor of the same k split in the launch.
 // Wide inputs per workgroup: a CU runs two workgroups; a full round of 512
 // takes 34, 45 and 56 us for 32, 48 and 64 inputs of 8 groups, one of up to
 // 256 (alone on their CU) 22, 30 and 37 us.  The least of the sum.
-Fp8MmPlan fp8_mm_plan(const Tensor& t, size_t rows, size_t n, size_t group_rows, const Tensor* t2 = nullptr,
-                      size_t rows2 = 0) {
+Fp8MmPlan fp8_mm_plan(const Tensor& t, size_t rows, size_t n, size_t group_rows, size_t rows2 = 0) {
     Fp8MmPlan p;
     p.kg = fp8_mm_groups(t, rows, n);
-    if (t2) p.kg2 = fp8_mm_groups(*t2, rows2, n);
-    if (n <= 16 || p.kg == 0 || (t2 && p.kg2 == 0)) return p;
-    if (rows < WH_FP8MMW_ROWS || (t2 && rows2 < WH_FP8MMW_ROWS) || (group_rows && group_rows < WH_FP8MMW_ROWS))
+    if (n <= 16 || p.kg == 0) return p;
+    if (rows < WH_FP8MMW_ROWS || (rows2 && rows2 < WH_FP8MMW_ROWS) || (group_rows && group_rows < WH_FP8MMW_ROWS))
         return p;
     const size_t G = t.cols / 128;
-    const size_t rb1 = (rows + WH_FP8MMW_ROWS - 1) / WH_FP8MMW_ROWS;
-    const size_t rb2 = t2 ? (rows2 + WH_FP8MMW_ROWS - 1) / WH_FP8MMW_ROWS : 0;
-    if ((rb1 + rb2) * ((n + 31) / 32) * G <= 1024 && (!t2 || p.kg == p.kg2)) return p;
+    const size_t rb = (rows + WH_FP8MMW_ROWS - 1) / WH_FP8MMW_ROWS + (rows2 + WH_FP8MMW_ROWS - 1) / WH_FP8MMW_ROWS;
+    if (rb * ((n + 31) / 32) * G <= 1024) return p;
     size_t best = SIZE_MAX;
     for (int kt = 2; kt <= 4; ++kt) {
         const size_t tbs = (n + 16 * kt - 1) / (16 * kt);
-        const size_t wgs = tbs * (rb1 * (G / p.kg) + (t2 ? rb2 * (G / p.kg2) : 0));
+        const size_t wgs = tbs * rb * (G / p.kg);
         const size_t tail = wgs % 512;
         const size_t cost = wgs / 512 * (12 + 11 * kt) + (tail == 0 ? 0 : tail <= 256 ? 7 + 15 * kt / 2 : 12 + 11 * kt);
         if (cost < best) {
@@ -802,20 +797,18 @@ Fp8MmPlan fp8_mm_plan(const Tensor& t, size_t rows, size_t n, size_t group_rows,
 // r0 + [g group_rows, (g + 1) group_rows) read input group g at
 // x + g * xg_stride.  One launch over (row block, k split, token block); with
 // `second`, its row blocks follow the first tensor's in the same launch
-// (the caller checks that the plan takes both: it is wide, or they have the
-// same k split).
+// (the caller checks that both take the same k split).
 int launch_fp8_mm(wh_ctx* c, const Tensor& t, size_t r0, size_t r1, const float* x, size_t n, size_t x_stride,
                   float* y, size_t y_stride, size_t group_rows, size_t xg_stride,
                   const Fp8MmSecond* second = nullptr) {
     const size_t rows = r1 - r0, rows2 = second ? second->r1 - second->r0 : 0, G = t.cols / 128;
-    const Fp8MmPlan plan = fp8_mm_plan(t, rows, n, group_rows, second ? second->t : nullptr, rows2);
+    const Fp8MmPlan plan = fp8_mm_plan(t, rows, n, group_rows, rows2);
     if (plan.kg == 0) return WH_UNSUPPORTED;
     const size_t row_block = plan.kt ? WH_FP8MMW_ROWS : WH_FP8MM_ROWS;
     const size_t tok_block = plan.kt ? 16 * (size_t)plan.kt : WH_FP8MM_TOK;
     const size_t rb1 = (rows + row_block - 1) / row_block, rb2 = (rows2 + row_block - 1) / row_block;
     const size_t rb = rb1 + rb2, tbs = (n + tok_block - 1) / tok_block;
-    const size_t kc = plan.kg * 128, S1 = G / plan.kg;
-    const size_t S2 = second && plan.kt ? G / plan.kg2 : S1, S = std::max(S1, S2);
+    const size_t kc = plan.kg * 128, S = G / plan.kg;
     const size_t rb128 = (rows + 127) / 128 + (rows2 + 127) / 128;
     if (rb128 * S > 65535 || tbs > 65535) return WH_UNSUPPORTED;
     if (S > 1) {
@@ -842,12 +835,9 @@ int launch_fp8_mm(wh_ctx* c, const Tensor& t, size_t r0, size_t r1, const float*
     a.xg_shift = group_rows ? log2_of(group_rows) : 31u;
     a.xg_stride = (uint32_t)xg_stride;
     a.kc = (uint32_t)kc;
-    a.splits = (uint32_t)S1;
+    a.splits = (uint32_t)S;
     a.row_blocks = (uint32_t)rb;
     a.rb_first = (uint32_t)rb1;
-    a.kc2 = (uint32_t)(second && plan.kt ? plan.kg2 * 128 : kc);
-    a.splits2 = (uint32_t)S2;
-    a.ws_splits = (uint32_t)S;
     if (second) {
         a.w2 = second->t->w;
         a.scales2 = second->t->s;
@@ -2875,18 +2865,17 @@ int wh_fp8_gemv_multi_pair_async(wh_ctx* c, wh_tensor w0, size_t row_start0, siz
     WH_HIP(hipSetDevice(c->device));
     const bool mm0 = !c->exact && n >= c->fp8_mm_min && fp8_mm_ok(*t0, row_start0, row_end0, 0);
     const bool mm1 = !c->exact && n >= c->fp8_mm_min && fp8_mm_ok(*t1, row_start1, row_end1, 0);
-    // one launch when both take the MFMA path (k_fp8_mm: with the same k split), the
+    // one launch when both take the MFMA path with the same k split, the
     // tensors agree in width, scale format, rows per scale row and special
     // codes, and neither output overlaps the inputs or the other output
     // (the two calls are ordered; where the order could show, they stay two)
     if (mm0 && mm1 && t0->cols == t1->cols && t0->scale_fmt == t1->scale_fmt && t0->special == t1->special &&
-        t0->rows / t0->scale_rows == t1->rows / t1->scale_rows && t0->scale_cols == t1->scale_cols) {
-        const Fp8MmPlan plan = fp8_mm_plan(*t0, row_end0 - row_start0, n, 0, t1, row_end1 - row_start1);
-        const bool one = plan.kt || plan.kg == plan.kg2;  // the wide kernel takes two k splits
+        t0->rows / t0->scale_rows == t1->rows / t1->scale_rows && t0->scale_cols == t1->scale_cols &&
+        fp8_mm_groups(*t0, row_end0 - row_start0, n) == fp8_mm_groups(*t1, row_end1 - row_start1, n)) {
         const uintptr_t x_lo = (uintptr_t)x_dev, x_hi = (uintptr_t)(x_dev + (n - 1) * x_stride + t0->cols);
         const uintptr_t a_lo = (uintptr_t)y0_dev, a_hi = (uintptr_t)(y0_dev + (n - 1) * y0_stride + (row_end0 - row_start0));
         const uintptr_t b_lo = (uintptr_t)y1_dev, b_hi = (uintptr_t)(y1_dev + (n - 1) * y1_stride + (row_end1 - row_start1));
-        if (one && !(a_lo < x_hi && x_lo < a_hi) && !(b_lo < x_hi && x_lo < b_hi) && !(a_lo < b_hi && b_lo < a_hi)) {
+        if (!(a_lo < x_hi && x_lo < a_hi) && !(b_lo < x_hi && x_lo < b_hi) && !(a_lo < b_hi && b_lo < a_hi)) {
             const Fp8MmSecond sec{t1, row_start1, row_end1, y1_dev, y1_stride};
             return launch_fp8_mm(c, *t0, row_start0, row_end0, x_dev, n, x_stride, y0_dev, y0_stride, 0, 0, &sec);
         }
