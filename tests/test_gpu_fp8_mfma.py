@@ -367,3 +367,15 @@ def test_pair_past_one_grid(ctx):
         ctx.device_free(p)
     for a, b in zip(*got):
         assert np.any(a) and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def test_more_inputs_than_a_grid_refused():
+    """More than 65535 tiles of 16 inputs (only the host entry point takes so
+    many) are refused, whichever kernel they would take."""
+    rows, cols, n = 256, 256, 65535 * 16 + 1
+    with wohper_amd.Context(0) as c:
+        c.set_exact_numerics(False)
+        t = c.store_fp8_synthetic(rows, cols, 3, 1, np.ones((2, 2), np.float32))
+        with pytest.raises(wohper_amd.DeepSeekV4KernelError) as e:
+            c.fp8_gemv_multi(t, np.zeros((n, cols), np.float32), 0, rows)
+        assert e.value.name == "Unsupported"

@@ -809,8 +809,9 @@ int launch_fp8_mm(wh_ctx* c, const Tensor& t, size_t r0, size_t r1, const float*
     const size_t rb1 = (rows + row_block - 1) / row_block, rb2 = (rows2 + row_block - 1) / row_block;
     const size_t rb = rb1 + rb2, tbs = (n + tok_block - 1) / tok_block;
     const size_t kc = plan.kg * 128, S = G / plan.kg;
+    // the limits of k_fp8_mm's grid, whichever kernel runs
     const size_t rb128 = (rows + 127) / 128 + (rows2 + 127) / 128;
-    if (rb128 * S > 65535 || tbs > 65535) return WH_UNSUPPORTED;
+    if (rb128 * S > 65535 || (n + WH_FP8MM_TOK - 1) / WH_FP8MM_TOK > 65535) return WH_UNSUPPORTED;
     if (S > 1) {
         WH_HIP(c->fp8mm_ws.ensure(tbs * rb * S * row_block * tok_block * sizeof(float), false));
         WH_HIP(c->fp8mm_cnt.ensure(tbs * rb * sizeof(uint32_t), true));
