@@ -762,10 +762,12 @@ struct Fp8MmPlan {
 // k split is k_fp8_mm's either way, so the results are too):
 //  - k_fp8_mm for at most 16 inputs, which it reads the weights once for, for
 //    tensors or input groups under a row block of 256, and where the work,
-//    counted in units of 256 rows x 32 inputs x 128 columns, is at most 1024:
-//    1024 x 4096 takes 10 us there for 64 inputs and 12 for 128 (wide: 14 to 18);
-//    32768 x 1024 and 4096 x 8192 the same in both for 32; at the next step, 40
-//    inputs, they take 22.6 and 29.8 us there and 20.6 and 25.0 us wide.
+//    counted in units of 256 rows x 16 inputs x 128 columns, is at most 2560:
+//    there 4096 x 4096 and 2048 x 8192 with 80 inputs take 23.3 and 25.2 us
+//    (wide 24.6 and 27.5), with 96 inputs, 3072 units, 27.5 and 29.8 (25.5 and
+//    28.1).  For widths without splits of 8 groups, whose workgroups gain
+//    most, 2048: 32768 x 256 with 160 inputs, 2560 units, takes 22.5 us there
+//    and 16.9 wide.
 // With rows2 more of a second tensor of the same k split in the launch.
 // Wide inputs per workgroup: a CU runs two workgroups; a full round of 512
 // takes 34, 45 and 56 us for 32, 48 and 64 inputs of 8 groups, one of up to
@@ -778,7 +780,7 @@ Fp8MmPlan fp8_mm_plan(const Tensor& t, size_t rows, size_t n, size_t group_rows,
         return p;
     const size_t G = t.cols / 128;
     const size_t rb = (rows + WH_FP8MMW_ROWS - 1) / WH_FP8MMW_ROWS + (rows2 + WH_FP8MMW_ROWS - 1) / WH_FP8MMW_ROWS;
-    if (rb * ((n + 31) / 32) * G <= 1024) return p;
+    if (rb * ((n + 15) / 16) * G <= (p.kg < 8 ? 2048u : 2560u)) return p;
     size_t best = SIZE_MAX;
     for (int kt = 2; kt <= 4; ++kt) {
         const size_t tbs = (n + 16 * kt - 1) / (16 * kt);
