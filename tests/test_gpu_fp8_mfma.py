@@ -379,20 +379,3 @@ def test_more_inputs_than_a_grid_refused():
         with pytest.raises(wohper_amd.DeepSeekV4KernelError) as e:
             c.fp8_gemv_multi(t, np.zeros((n, cols), np.float32), 0, rows)
         assert e.value.name == "Unsupported"
-
-
-def test_wide_kernel_from_its_gain_on_time(ctx):
-    """2048 x 8192: 80 inputs are five tiles of the narrow kernel (25.2 us) and
-    less than the 96 that three blocks of the wide one take (28.1 us; 80 there
-    27.5)."""
-    rows, cols = 2048, 8192
-    t = ctx.store_fp8_synthetic(rows, cols, 3, 1, np.full((rows // 128, cols // 128), 2.0 ** -10, np.float32))
-    x = np.random.default_rng(5).standard_normal((96, cols)).astype(np.float32)
-    xd, y = ctx.device_alloc(x.nbytes), ctx.device_alloc(4 * 96 * rows)
-    ctx.to_device(xd, x)
-    us = {n: _graph_us(ctx, lambda: ctx.fp8_gemv_multi_async(t, 0, rows, xd, n, cols, y, rows)) for n in (80, 96)}
-    print(f"{rows} x {cols}: 80 inputs {us[80]:.1f} us, 96 inputs {us[96]:.1f} us")
-    ctx.release(t)
-    ctx.device_free(xd)
-    ctx.device_free(y)
-    assert us[80] <= 0.95 * us[96]
