@@ -127,3 +127,51 @@ def test_multi_exact_pair_and_groups(ctx, oracle):
     ctx.device_free(yd)
     for t in (ta, tk, to):
         ctx.release(t)
+
+
+@pytest.mark.parametrize("rows,cols,n,r0,r1,ue8m0,special", [
+    (4096, 4096, 2, 0, 4089, True, True), (4096, 2048, 6, 16, 4096, False, False),
+    (4096, 1024, 13, 0, 4096, True, False),     # one round of 16-row tiles
+    (6144, 2048, 12, 16, 6137, False, True), (8192, 2048, 13, 16, 8185, True, False),   # two, a partial last one
+    (6144, 2048, 24, 16, 6137, True, True), (16384, 1024, 15, 0, 16377, False, False),  # 32-row tiles
+    (32768, 1024, 15, 0, 32761, False, False)])
+def test_multi_exact_matrix_instructions_full_rounds(ctx, oracle, rows, cols, n, r0, r1, ue8m0, special):
+    """Products that the one-term matrix instructions take: rounds of 256
+    workgroups that are full enough, with partial tiles of rows and inputs."""
+    t, w, scales = _tensor(ctx, rows, cols, rows + n, ue8m0, special)
+    xs = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    xs[0] *= np.float32(2.0 ** -126)
+    xs[n - 1] *= np.float32(1e30)
+    ys = _run(ctx, t, xs, r0, r1)
+    want = oracle.fp8_gemv_rows_multi(w, rows, cols, scales, rows // 128, cols // 128, xs, r0, r1)
+    assert np.array_equal(bits(ys), bits(np.stack(want)))
+    ctx.release(t)
+
+
+@pytest.mark.parametrize("rows,cols,n,most", [(5120, 2048, 9, 1.15), (6144, 3072, 9, 1.12), (5120, 1024, 13, 1.3)])
+def test_multi_exact_time_follows_inputs(ctx, rows, cols, n, most):
+    """Products that fill less than half of a round of the matrix
+    instructions' workgroups stay with the vector kernel: one more input than
+    a whole block of it costs 1.07, 1.04 and 1.19 times as much, not the 1.31,
+    1.24 and 1.41 times of a tile of 16."""
+    t = ctx.store_fp8_synthetic(rows, cols, 3, 1, np.full((rows // 128, cols // 128), 2.0 ** -10, np.float32))
+    x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    xd, y = ctx.device_alloc(x.nbytes), ctx.device_alloc(4 * n * rows)
+    ctx.to_device(xd, x)
+    us = {}
+    for k in (n - 1, n):
+        ctx.fp8_gemv_multi_async(t, 0, rows, xd, k, cols, y, rows)
+        ctx.synchronize()
+        g = ctx.graph_capture(lambda: [ctx.fp8_gemv_multi_async(t, 0, rows, xd, k, cols, y, rows) for _ in range(20)])
+        v = []
+        for _ in range(6):
+            ctx.timer_start()
+            ctx.graph_launch(g)
+            v.append(ctx.timer_stop() / 20)
+        ctx.graph_release(g)
+        us[k] = min(v)
+    print(f"{rows} x {cols}: {n - 1} inputs {us[n - 1]:.2f} us, {n} inputs {us[n]:.2f} us")
+    ctx.release(t)
+    ctx.device_free(xd)
+    ctx.device_free(y)
+    assert us[n] <= most * us[n - 1]

@@ -503,6 +503,30 @@ bool fp8_split_k(const Tensor& t) {
     return t.fast && (t.cols / 128) % 8 == 0 && fp8_sk_lds(t.cols) <= g_max_lds && is_pow2(t.rows / t.scale_rows);
 }
 
+// Whether k_fp8_exact_mm takes a product of `work` = inputs x rows in `wgs`
+// workgroups of `per` rows x 16 inputs, against the vector kernels.  Its time
+// goes by rounds of 256 workgroups, that of k_fp8_gemv_multi by inputs, so the
+// rounds have to be full enough (us, this against k_fp8_gemv_multi):
+//  - one round of 16-row tiles (at most 4096 rows): 8.3 against 7.6 to 8.1 for
+//    2 to 5 inputs of 4096 x 2048, 8.3 and 9.6 for 8; from 4096 columns on
+//    always, 4096 x 8192 22.7 and 25.1 for 2 inputs, 21.6 and 34.6 for 16;
+//  - else over half full: 5120 x 2048 with 9, 12 and 13 inputs (0.35, 0.47 and
+//    0.51 full) 13.3 against 10.8, 11.4 and 13.3, 6144 x 2048 with 12 (0.56)
+//    13.5 and 15.0; 16384 x 4096 with 8 (0.5) and 9 36.1 against 31.8 and 50.1.
+//    From three rounds on the vector kernel's are full too: under 4096 columns
+//    over 0.66, 12288 x 2048 with 17, 21 and 24 (0.53, 0.66 and 0.75) 30.2,
+//    29.7 and 29.9 against 27.2, 28.1 and 31.8;
+//  - 1024 columns, where a workgroup's first loads are most of its time, over
+//    0.74, from four rounds on 0.82, and not in three rounds: 6144 x 1024 with
+//    16 (0.75) 9.5 and 10.4, with 48 in three rounds (0.75) 20.0 and 18.3; 32768
+//    with 13 (0.81) 27.1 and 25.9, with 16 27.1 and 28.9.
+bool exact_mm_faster(size_t work, size_t wgs, size_t per, size_t cols) {
+    const size_t rounds = (wgs + 255) / 256, full = rounds * 256 * per * 16;
+    if (cols <= 1024) return rounds != 3 && 100 * work > (rounds > 3 ? 82 : 74) * full;
+    if (per == 16 && rounds == 1) return cols >= 4096 || 16 * work > 5 * full;
+    return 100 * work > (rounds > 2 && cols < 4096 ? 66 : 50) * full;
+}
+
 // x_group_rows / x_group_stride: row groups with their own input (split-K
 // path only; see wh_fp8_args).
 // order_free: with exact numerics off the order-free kernel may run (the
@@ -597,25 +621,20 @@ int launch_fp8(wh_ctx* c, const Tensor& t, size_t r0, size_t r1, const float* x,
         }
     }
     // several inputs in the reference's order on matrix instructions
-    // (k_fp8_exact_mm).  Its time goes by tiles of 16 inputs, that of the vector
-    // kernel below by inputs, so a tile has to be full enough; one tile against
-    // the vector kernel, us: 4096 x 8192 22.2 (2 to 5 inputs 26, 8 inputs 31, 13
-    // 36), 8192 x 4096 23.6 (5 inputs 18, 8 22, 13 32), 32768 x 1024, where a
-    // workgroup's first loads are most of its time, 27.9 (8 inputs 18, 13 30).
-    // Below 4096 rows the per-input kernel's wider grid is faster.  Two row
-    // tiles a wave where 32-row workgroups still cover the chip's 256 CUs
+    // (k_fp8_exact_mm), 16 inputs a tile: two row tiles a wave where 32-row
+    // workgroups still cover the chip's 256 CUs
     const size_t xrows = (r1 - r0) + (t2 ? r1_2 - r0_2 : 0), tiles = (n_batch + 15) / 16;
-    const size_t tile_min = t.cols <= 1024 ? 13 : xrows > 4096 ? 9 : 2;
+    const bool pair = xrows / 32 * tiles >= 256;
+    const size_t per = pair ? 32 : 16, b1 = (r1 - r0 + per - 1) / per, b2 = t2 ? (r1_2 - r0_2 + per - 1) / per : 0;
     const auto tile_ok = [](const Tensor& m, size_t row) { return row % 16 == 0 && (m.rows / m.scale_rows) % 16 == 0; };
-    if (n_batch >= 2 && xrows >= 4096 && n_batch >= tile_min * tiles && fp8_split_k(t) && t.cols % (256 * WH_FP8_XMM_GROUPS) == 0 && tile_ok(t, r0) &&
+    if (n_batch >= 2 && xrows >= 4096 && exact_mm_faster(n_batch * xrows, (b1 + b2) * tiles, per, t.cols) && fp8_split_k(t) &&
+        t.cols % (256 * WH_FP8_XMM_GROUPS) == 0 && tile_ok(t, r0) &&
         (!t2 || (fp8_split_k(*t2) && t2->cols == t.cols && t2->special == t.special &&
                  t2->scale_fmt == t.scale_fmt && tile_ok(*t2, r0_2))) &&
         (!x_group_rows || (x_group_rows % 32 == 0 && x_group_stride % 4 == 0)) && x_stride % 4 == 0 &&
         !((uintptr_t)x & 15) && tiles <= 65535) {
-        const bool pair = xrows / 32 * tiles >= 256;
-        const size_t per = pair ? 32 : 16, b1 = (r1 - r0 + per - 1) / per;
         if (t2) a.blocks1 = (uint32_t)b1;
-        dim3 grid((unsigned)(b1 + (t2 ? (r1_2 - r0_2 + per - 1) / per : 0)), (unsigned)tiles);
+        dim3 grid((unsigned)(b1 + b2), (unsigned)tiles);
         const uint32_t n_in = (uint32_t)n_batch;
         auto go = [&](auto special, auto is_u8) {
             constexpr bool kSp = decltype(special)::value, kU8 = decltype(is_u8)::value;
