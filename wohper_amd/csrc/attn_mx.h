@@ -33,37 +33,30 @@ struct wh_attn_f4 {  // four floats at any float's alignment
 // sides), LDS only joins the quarters.  For few positions, which 16 heads a
 // workgroup leave enough workgroups; a batch takes k_attn_scores_mx_tile.
 __global__ void __launch_bounds__(256) k_attn_scores_mx(wh_attn_args a) {
-    constexpr int kH = 1;  // 16-head tiles
     constexpr int kS = 4;  // 16-dim steps requested together
-    constexpr int kE = 2 * kH, kLanes = 32 / kE;
-    __shared__ __align__(16) float red[4][2 * kH][256];
+    __shared__ __align__(16) float red[4][2][256];
     const wh_attn_pos v = wh_attn_resolve(a, blockIdx.z);
     const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63, col = lane & 15, q = lane >> 4;
     const uint32_t nk = v.n_win + v.n_comp, hd = a.head_dim, n_s = hd / 64;
-    const uint32_t j0 = blockIdx.x * WH_ATTN_MX_KEYS, h0 = blockIdx.y * (16 * kH);
+    const uint32_t j0 = blockIdx.x * WH_ATTN_MX_KEYS, h0 = blockIdx.y * 16;
     if (j0 >= nk) return;  // a batched launch's grid covers its longest key list
     const uint32_t base = wave * (hd / 4) + 4 * q;
-    const float *qp[kH], *kp[2];
-#pragma unroll
-    for (int h = 0; h < kH; ++h) qp[h] = v.q + (size_t)min(h0 + 16 * h + col, a.heads - 1) * hd + base;
+    const float* const qp = v.q + (size_t)min(h0 + col, a.heads - 1) * hd + base;
+    const float* kp[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) kp[k] = wh_attn_key(a, v, min(j0 + 16 * k + col, nk - 1)) + base;
-    wh_f4 qv[2][kS][kH], kv[2][kS][2];
+    wh_f4 qv[2][kS], kv[2][kS][2];
     auto request = [&](int b, uint32_t s0) {
 #pragma unroll
         for (int s = 0; s < kS; ++s) {
             const uint32_t o = 16 * min(s0 + s, n_s - 1);
-#pragma unroll
-            for (int h = 0; h < kH; ++h) qv[b][s][h] = *(const wh_f4*)(qp[h] + o);
+            qv[b][s] = *(const wh_f4*)(qp + o);
 #pragma unroll
             for (int k = 0; k < 2; ++k) kv[b][s][k] = *(const wh_f4*)(kp[k] + o);
         }
     };
-    wh_f4 acc[kH][2];
-#pragma unroll
-    for (int h = 0; h < kH; ++h)
-#pragma unroll
-        for (int k = 0; k < 2; ++k) acc[h][k] = (wh_f4){0.0f, 0.0f, 0.0f, 0.0f};
+    wh_f4 acc[2];
+    acc[0] = acc[1] = (wh_f4){0.0f, 0.0f, 0.0f, 0.0f};
     auto multiply = [&](int b, uint32_t s0) {
 #pragma unroll
         for (int s = 0; s < kS; ++s) {
@@ -71,11 +64,8 @@ __global__ void __launch_bounds__(256) k_attn_scores_mx(wh_attn_args a) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int h = 0; h < kH; ++h)
-#pragma unroll
-                        for (int k = 0; k < 2; ++k)
-                            acc[h][k] =
-                                __builtin_amdgcn_mfma_f32_16x16x4f32(qv[b][s][h][i], kv[b][s][k][i], acc[h][k], 0, 0, 0);
+                    for (int k = 0; k < 2; ++k)
+                        acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[b][s][i], kv[b][s][k][i], acc[k], 0, 0, 0);
             }
         }
     };
@@ -88,33 +78,31 @@ __global__ void __launch_bounds__(256) k_attn_scores_mx(wh_attn_args a) {
     }
     // D[4 q + r][col]: head, key
 #pragma unroll
-    for (int h = 0; h < kH; ++h)
+    for (int k = 0; k < 2; ++k)
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) red[wave][2 * h + k][(4 * q + r) * 16 + col] = acc[h][k][r];
+        for (int r = 0; r < 4; ++r) red[wave][k][(4 * q + r) * 16 + col] = acc[k][r];
     __syncthreads();
-    // thread: kE keys of one head, kLanes threads a head
-    const uint32_t hl = t / kLanes, e0 = (t % kLanes) * kE, h = h0 + hl;
-    const uint32_t tile = 2 * (hl >> 4) + (e0 >> 4), at = (hl & 15) * 16 + (e0 & 15);
+    // thread: two keys of one head, 16 threads a head
+    const uint32_t e0 = (t & 15) * 2, h = h0 + (t >> 4);
+    const uint32_t tile = e0 >> 4, at = (t >> 4) * 16 + (e0 & 15);
     const float ninf = -__uint_as_float(0x7f800000u);
-    float s[kE], mx = ninf;
+    float s[2], mx = ninf;
 #pragma unroll
-    for (int e = 0; e < kE; ++e) {
+    for (int e = 0; e < 2; ++e) {
         const float d = ((red[0][tile][at + e] + red[1][tile][at + e]) + (red[2][tile][at + e] + red[3][tile][at + e]));
         s[e] = d * a.scale;
         mx = fmaxf(mx, j0 + e0 + e < nk ? s[e] : ninf);
     }
 #pragma unroll
-    for (int off = kLanes / 2; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    for (int off = 8; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
     const float ref = mx == ninf ? 0.0f : mx;
     if (h >= a.heads) return;
 #pragma unroll
-    for (int e = 0; e < kE; ++e) {
+    for (int e = 0; e < 2; ++e) {
         const float w = wh_expf_glibc(s[e] - ref, kExpTab, kExpfExc, WH_EXPF_EXC_COUNT);
         if (j0 + e0 + e < nk) v.scores[(size_t)h * nk + j0 + e0 + e] = w;
     }
-    if (t % kLanes == 0) a.tile_max[((size_t)blockIdx.z * a.heads + h) * WH_ATTN_MX_TILES + blockIdx.x] = mx;
+    if ((t & 15) == 0) a.tile_max[((size_t)blockIdx.z * a.heads + h) * WH_ATTN_MX_TILES + blockIdx.x] = mx;
 }
 
 // k_attn_scores_mx for a batch that fills the chip with 32 heads x 64 keys a
