@@ -12,9 +12,11 @@ import numpy as np
 import pytest
 
 from parity_util import bits
-from test_gpu_decode_layer import HC, Dev, _setup
-from test_gpu_mla import HEAD_DIM
+from test_gpu_decode_layer import EPS, HC, ITERS, LAYER, N_EXP, Dev, _setup
+from test_gpu_mhc import _params
+from test_gpu_mla import GROUPS, HEAD_DIM, HEADS, NOPE, O_LORA, Q_LORA, ROPE
 import wohper_amd
+from wohper_amd import model_format as mf
 from wohper_amd import workloads as wl
 
 pytestmark = pytest.mark.gpu
@@ -135,6 +137,96 @@ def test_decode_layer_batch_order_free_many(ctx, oracle, dev):
     assert float(np.median(rel)) <= 3e-2
     for t in handles.values():
         ctx.release(t)
+
+
+def _store_router(ctx, layer, gate, bias):
+    blk = [mf.SyntheticTensor(f"layers.{layer}.ffn.gate.weight", 9, gate.shape, gate.tobytes(), 11, 2404)]
+    if bias is not None:
+        blk.append(mf.SyntheticTensor(f"layers.{layer}.ffn.gate.bias", 9, bias.shape, bias.tobytes(), 12, 2405))
+    ctx.store_router(layer, mf.build_synthetic_quant_block(blk), wl.HIDDEN)
+
+
+@pytest.mark.parametrize("kind", ["ties", "ties_no_bias", "nan_inf_bias", "zero_gate"])
+def test_decode_layer_batch_router_ties(ctx, oracle, dev, kind):
+    """Exact numerics: the router of 33 positions on matrix instructions
+    against the one-launch router of calls of at most four, bit for bit, with
+    equal keys inside the selected set and across its boundary, biases of NaN
+    and both infinities (the key of a selection, not its weight), and a gate
+    of zeros, whose keys are all the same."""
+    ctx.set_exact_numerics(True)
+    L, _, handles = _setup(ctx, oracle, dev)
+    n, ld = 33, HEAD_DIM
+    rng = np.random.default_rng(29)
+    gate = (rng.standard_normal((N_EXP, wl.HIDDEN)).astype(np.float32) * 0.02).view(np.uint32) >> 16
+    gate = gate.astype(np.uint16)
+    bias = (rng.standard_normal(N_EXP) * 0.05).astype(np.float32)
+    if kind.startswith("ties"):  # four rows to a key, so six cut a group
+        gate, bias = gate[np.arange(N_EXP) % 8], bias[np.arange(N_EXP) % 8]
+    elif kind == "nan_inf_bias":
+        bias[[3, 17]], bias[[5, 30]], bias[[0, 9, 31]] = np.nan, np.inf, -np.inf
+    else:
+        gate[:] = 0
+        bias[:] = 0.25
+    _store_router(ctx, LAYER, gate, None if kind == "ties_no_bias" else bias)
+    kv0 = (rng.standard_normal((n + 3, ld)) * 0.3).astype(np.float32)
+    positions = list(range(3, 3 + n))
+    h0 = (rng.standard_normal((n, HC * wl.HIDDEN)) * 0.5).astype(np.float32)
+    got, got_kv = _run(ctx, dev, L, h0, positions, kv0, ld)
+    want, kv = np.empty_like(got), kv0
+    for i in range(0, n, 4):
+        want[i:i + 4], kv = _run(ctx, dev, L, h0[i:i + 4], positions[i:i + 4], kv, ld)
+    assert np.array_equal(bits(got_kv), bits(kv)) and np.all(np.isfinite(got))
+    for i in range(n):
+        assert np.array_equal(bits(got[i]), bits(want[i])), i
+    for t in handles.values():
+        ctx.release(t)
+
+
+def test_decode_layer_batch_hc_sums_bits(ctx, dev):
+    """Exact numerics off: hc_pre's sums of four streams a workgroup (from 32
+    positions on) are the one-stream kernel's bits.  In a layer whose sub-block
+    outputs do not depend on its inputs (a cache of ones under zero queries and
+    zero new rows through one-hot output weights; experts of 2^-126, which add
+    zero) the hidden state that comes out is post and comb, so the sums and
+    their normalisation, times values that are the same in any call."""
+    layer, n_exp, rng = LAYER + 1, 16, np.random.default_rng(31)
+    shapes = {"wq_a": (Q_LORA, wl.HIDDEN), "wq_b": (HEADS * HEAD_DIM, Q_LORA), "wkv": (HEAD_DIM, wl.HIDDEN),
+              "wo_a": (GROUPS * O_LORA, HEADS * HEAD_DIM // GROUPS), "wo_b": (wl.HIDDEN, GROUPS * O_LORA)}
+    t = {}
+    for k, (r, c) in shapes.items():
+        w = np.zeros((r, c), np.uint8)
+        if k in ("wo_a", "wo_b"):
+            w[np.arange(r), rng.integers(0, c, r) // HEAD_DIM * HEAD_DIM + rng.integers(0, NOPE, r)] = 0x38
+        t[k] = ctx.store_fp8(w, r, c, np.ones((r // 128, c // 128), np.float32), r // 128, c // 128, wohper_amd.SCALE_F32)
+    for e in range(n_exp + 1):
+        ctx.store_expert_synthetic(layer, e, wl.HIDDEN, wl.INTER, 5, 1, 1)
+    gate = (rng.standard_normal((n_exp, wl.HIDDEN)).astype(np.float32) * 0.02).view(np.uint32) >> 16
+    _store_router(ctx, layer, gate.astype(np.uint16), None)
+    L = wohper_amd.WhMhcLayer()
+    L.hc, L.hidden, L.sinkhorn_iters, L.hc_eps = HC, wl.HIDDEN, ITERS, EPS
+    L.hc_attn_fn, L.hc_attn_scale, L.hc_attn_base = (dev.put(a) for a in _params(rng, HC, wl.HIDDEN))
+    L.hc_ffn_fn, L.hc_ffn_scale, L.hc_ffn_base = (dev.put(a) for a in _params(rng, HC, wl.HIDDEN))
+    L.attn = wohper_amd.WhMlaLayer(0, HEADS, NOPE, ROPE, GROUPS, O_LORA, t["wq_a"], t["wq_b"], t["wkv"], t["wo_a"],
+                                   t["wo_b"], None, None, dev.put(np.zeros(HEADS, np.float32)))
+    L.layer_id, L.active, L.available_dev, L.n_available = layer, 6, None, 0
+    L.route = wohper_amd.Context.route_options(wohper_amd.ROUTER_SQRT_SOFTPLUS, 1.5)
+    L.shared_layer, L.shared_expert = layer, n_exp
+    n, ld = 35, HEAD_DIM
+    kv0 = np.ones((100 + n, ld), np.float32)
+    h0 = (rng.standard_normal((n, HC * wl.HIDDEN)) * 0.5).astype(np.float32)
+    positions = list(range(100, 100 + n))
+    ctx.set_exact_numerics(False)
+    want, kv = np.empty_like(h0), kv0
+    for i in range(0, n, 8):
+        want[i:i + 8], kv = _run(ctx, dev, L, h0[i:i + 8], positions[i:i + 8], kv, ld)
+    # the layer's outputs reach the hidden state, and differ between its copies
+    assert np.all(np.isfinite(want)) and np.abs(want).max() > 0.1
+    for k in (32, 33, 34, 35):
+        got, _ = _run(ctx, dev, L, h0[:k], positions[:k], kv0, ld)
+        for i in range(k):
+            assert np.array_equal(bits(got[i]), bits(want[i])), (k, i, int(np.count_nonzero(got[i] != want[i])))
+    for h in t.values():
+        ctx.release(h)
 
 
 def test_decode_layer_batch_errors(ctx, oracle, dev):

@@ -229,14 +229,17 @@ def test_pair_equals_two_multi_calls(ctx, oracle, exact):
 
 
 @pytest.mark.parametrize("rows,cols,n,r0,r1,special", [
-    (2304, 8192, 33, 0, 2304, False),     # 32-input blocks, the second with one input
-    (2560, 8192, 40, 16, 2544, True),     # a row range off the 64- and 256-row grids, all codes
-    (4096, 2048, 144, 0, 4096, False),    # 48-input blocks
-    (4096, 4096, 250, 0, 4080, False),    # 64-input blocks, the last partial
+    (2304, 8192, 65, 0, 2304, False),     # 32-input blocks, the last with one input
+    (2560, 8192, 80, 16, 2544, True),     # a row range off the 64- and 256-row grids, all codes
+    (4096, 2048, 192, 0, 4096, False),    # whole blocks
+    (4096, 4096, 250, 0, 4080, False),    # two rounds of workgroups, the last block partial
+    (4096, 8192, 80, 16, 4090, True),     # 48-input blocks, the last partial
+    (8192, 4096, 220, 0, 8192, False),    # 64-input blocks, the last partial
 ])
 def test_fp8_mfma_wide_against_oracle(ctx, oracle, rows, cols, n, r0, r1, special):
     """k_fp8_mm_wide at the edges of its row and input blocks, within the
-    bound of any fp32 summation order."""
+    bound of any fp32 summation order: blocks of 32 inputs but for the last
+    two cases."""
     case = wl.fp8_gemv_case(rows, cols, seed=rows + n)
     w = case.w.copy()
     if special:
@@ -254,7 +257,7 @@ def test_fp8_mfma_wide_against_oracle(ctx, oracle, rows, cols, n, r0, r1, specia
 def test_fp8_mfma_wide_one_hot_exact(ctx, oracle, ue8m0):
     """One one-hot input per column, in one call: every weight and scale comes
     out exactly at its own row, column and input."""
-    rows, cols = 1280, 1024
+    rows, cols = 1536, 1024
     rng = np.random.default_rng(5)
     w = rng.integers(0, 256, (rows, cols)).astype(np.uint8)
     e = rng.integers(-6, 3, (rows // 128, cols // 128))
@@ -270,8 +273,9 @@ def test_fp8_mfma_wide_one_hot_exact(ctx, oracle, ue8m0):
 
 @pytest.mark.parametrize("n", [49, 128, 193])
 def test_fp8_mfma_wide_pair_and_groups(ctx, n):
-    """wq_a + wkv in one launch with two k splits, and wo_a's row groups, are
-    the single calls bit for bit."""
+    """wq_a + wkv as a pair, which their two k splits make two launches, are the
+    single calls bit for bit, wo_a's row groups (blocks of 32 and 64 inputs)
+    up to the sums' order."""
     cols = 4096
     rng = np.random.default_rng(n)
     cases = [wl.fp8_gemv_case(r, cols, seed=r + n) for r in (1024, 512, 8192)]
@@ -306,6 +310,60 @@ def test_fp8_mfma_wide_pair_and_groups(ctx, n):
         ctx.release(t)
     ctx.device_free(xd)
     ctx.device_free(yd)
+
+
+@pytest.mark.parametrize("rows,cols,n,r0,r1,special,ue8m0", [
+    (4096, 8192, 33, 0, 4096, False, True), (8192, 4096, 40, 32, 8181, True, False),      # 32-input blocks
+    (4096, 8192, 80, 16, 4090, True, False), (8192, 4096, 131, 32, 8192, False, True),    # 48
+    (32768, 1024, 165, 16, 32765, True, True),                                            # 48, no k split
+    (4096, 8192, 193, 16, 4090, False, False), (8192, 4096, 220, 0, 8181, True, True),    # 64
+    (32768, 1024, 222, 0, 32768, False, True)])                                           # 64, no k split
+def test_fp8_mfma_wide_is_narrow_bits(ctx, rows, cols, n, r0, r1, special, ue8m0):
+    """k_fp8_mm_wide with 32, 48 and 64 inputs a workgroup, partial last blocks
+    of inputs and rows, gives k_fp8_mm's bits: calls of at most 16 inputs stay
+    with that, and tensors of 256 or more (128-row block, split of 8 groups)
+    pairs take the same k split for any number of inputs."""
+    assert (r1 - r0 + 127) // 128 * (cols // 1024) >= 256
+    rng = np.random.default_rng(rows + n)
+    w = rng.integers(0, 256, (rows, cols), dtype=np.uint8)
+    if not special:
+        w[(w & 0x7F) == 0x7F] = 0x70
+    e = rng.integers(-8, -3, (rows // 128, cols // 128))
+    t = ctx.store_fp8(w, rows, cols, (e + 127).astype(np.uint8) if ue8m0 else np.exp2(e).astype(np.float32) * 1.25,
+                      rows // 128, cols // 128, wohper_amd.SCALE_UE8M0 if ue8m0 else wohper_amd.SCALE_F32)
+    xs = rng.standard_normal((n, cols)).astype(np.float32)
+    got = run_multi(ctx, t, xs, r0, r1, cols)
+    for i in [*range(0, n - 16, 16), n - 16]:  # under 4 inputs take another kernel
+        want = run_multi(ctx, t, xs[i:i + 16], r0, r1, cols)
+        assert np.any(want) and np.array_equal(got[i:i + 16].view(np.uint32), want.view(np.uint32)), i
+    ctx.release(t)
+
+
+@pytest.mark.parametrize("n", [49, 90])
+def test_fp8_mfma_wide_pair_of_one_split(ctx, n):
+    """Two tensors of one k split in one launch of k_fp8_mm_wide (32 and 48
+    inputs a workgroup), the second a row range, twice: the single calls' bits
+    and the arrival counters back at zero."""
+    rows, cols, r0 = 8192, 4096, 16
+    ts = [ctx.store_fp8_synthetic(rows, cols, 3, k, np.full((rows // 128, cols // 128), 2.0 ** -10, np.float32))
+          for k in (1, 2)]
+    x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    want = [np.empty((n, rows - r), np.float32) for r in (0, r0)]
+    for w, t, r in zip(want, ts, (0, r0)):
+        for i in [*range(0, n - 16, 16), n - 16]:  # under 4 inputs take another kernel
+            w[i:i + 16] = run_multi(ctx, t, x[i:i + 16], r, rows, cols)
+    xd, y = ctx.device_alloc(x.nbytes), [ctx.device_alloc(w.nbytes) for w in want]
+    ctx.to_device(xd, x)
+    for _ in range(2):
+        ctx.fp8_gemv_multi_pair_async(ts[0], 0, rows, y[0], rows, ts[1], r0, rows, y[1], rows - r0, xd, n, cols)
+        for w, p in zip(want, y):
+            got = np.empty_like(w)
+            ctx.from_device(got, p)
+            assert np.array_equal(got.view(np.uint32), w.view(np.uint32))
+    for t in ts:
+        ctx.release(t)
+    for p in (xd, *y):
+        ctx.device_free(p)
 
 
 def _graph_us(ctx, fn, reps=20):

@@ -179,6 +179,33 @@ def test_window_attention_shapes_bit_exact(ctx, oracle, dev, heads, hd, nope, pa
     assert np.array_equal(bits(dev.get(outp, (heads, hd))), bits(want))
 
 
+@pytest.mark.parametrize("heads,hd,nope,pairs", [(131, 1024, 960, 32), (257, 512, 448, 32), (515, 1024, 960, 32)])
+@pytest.mark.parametrize("n_comp", [1919, 1920])
+def test_window_attention_head_groups_bit_exact(ctx, oracle, dev, heads, hd, nope, pairs, n_comp):
+    """Two heads a wave for the scores and the weighted sums, four and two, and
+    four, each with a last group that is not full."""
+    test_window_attention_shapes_bit_exact(ctx, oracle, dev, heads, hd, nope, pairs, 128, n_comp)
+
+
+@pytest.mark.parametrize("rows", [16, 17, 1023, 1024, 1025])
+def test_rms_norm_tree_rows_of_512(ctx, dev, rows):
+    """Exact numerics off: rows of 512 without weights, one wave each, are the
+    row kernel's bits, which a call with weights of one takes."""
+    rng = np.random.default_rng(rows)
+    x = (rng.standard_normal((rows, 512)) * np.exp2(rng.integers(-6, 6, (rows, 1)))).astype(np.float32)
+    xp, yp, ones = dev.put(x), dev.empty(x.nbytes), dev.put(np.full(512, 0x3F80, np.uint16))
+    got = []
+    ctx.set_exact_numerics(False)
+    try:
+        for w in (0, ones):
+            ctx.rms_norm_async(xp, yp, rows, 512, w)
+            ctx.synchronize()
+            got.append(dev.get(yp, (rows, 512)))
+    finally:
+        ctx.set_exact_numerics(True)
+    assert np.any(got[0]) and np.array_equal(bits(got[0]), bits(got[1]))
+
+
 def _order_free_attention(ctx, dev, q, win, comp, sk, inv, nope, pairs, pos):
     heads, hd = q.shape
     nk = len(win) + len(comp)

@@ -106,9 +106,9 @@ def test_mla_batch_compressed_layer(ctx, oracle, dev):
 
 
 def test_mla_batch_many_positions(ctx, dev):
-    """35 positions (more than one launch's worth) with key lists from a few
-    rows to 700, so that one launch holds short and long ones: bit for bit the
-    single-token layer's outputs."""
+    """35 positions in one launch, with key lists from a few rows to 700, so
+    that it holds short and long ones: bit for bit the single-token layer's
+    outputs."""
     L, host, qn, kn, sink, handles = _layer(ctx, dev, 2)
     cap, ld = 240, HEAD_DIM
     rng = np.random.default_rng(14)
@@ -122,6 +122,82 @@ def test_mla_batch_many_positions(ctx, dev):
     assert np.array_equal(bits(got_cache), bits(want_cache))
     assert np.array_equal(bits(got), bits(want))
     for h in handles.values():
+        ctx.release(h)
+
+
+def test_mla_batch_two_launches(ctx, dev):
+    """131 positions, three more than one launch of the rows and the window
+    attention takes, with uneven compressed lists: at the first positions and
+    about the launches' edge bit for bit the single-token layer over the
+    batch's cache, whose rows up to a position are that position's."""
+    ctx.set_exact_numerics(True)
+    L, host, qn, kn, sink, handles = _layer(ctx, dev, 2)
+    n, cap, ld = 131, 400, HEAD_DIM
+    rng = np.random.default_rng(15)
+    cache0 = (rng.standard_normal((cap, ld)) * 0.3).astype(np.float32)
+    positions = list(range(3, 3 + 18)) + list(range(200, 200 + n - 18))
+    comp = dev.put((rng.standard_normal((700, HEAD_DIM)) * 0.3).astype(np.float32))
+    comps = [(comp + 4 * HEAD_DIM * int(o), int(k)) for o, k in zip(rng.integers(0, 300, n), rng.integers(1, 401, n))]
+    xs = rng.standard_normal((n, wl.HIDDEN)).astype(np.float32)
+    got, cache = _batch(ctx, dev, L, xs, positions, cache0, ld, comps)
+    for i in (0, 1, 17, 18, 126, 127, 128, 129, 130):
+        want, after = _sequential(ctx, dev, L, xs[i:i + 1], positions[i:i + 1], cache, ld, comps[i:i + 1])
+        assert np.array_equal(bits(after), bits(cache)), i
+        assert np.array_equal(bits(got[i]), bits(want[0])), i
+    for h in handles.values():
+        ctx.release(h)
+
+
+def _one_hot(ctx, rng, rows, cols):
+    """A resident matrix whose rows pick one column each, plus or minus it:
+    one product a row, the same bits in any order of summation."""
+    w = np.zeros((rows, cols), np.uint8)
+    pick = np.concatenate([rng.permutation(cols) for _ in range(-(-rows // cols))])[:rows]
+    w[np.arange(rows), pick] = rng.choice(np.array([0x38, 0xB8], np.uint8), rows)
+    return ctx.store_fp8(w, rows, cols, np.ones((rows // 128, cols // 128), np.float32), rows // 128, cols // 128,
+                         wohper_amd.SCALE_F32)
+
+
+@pytest.mark.parametrize("heads", [64, 48])
+@pytest.mark.parametrize("n", [5, 17, 33, 131])
+def test_mla_batch_order_free_window_alone(ctx, dev, heads, n):
+    """The order-free window kernels of a batch (from 16 positions on 32 heads
+    x 64 dims a workgroup, 48 heads with half a last one, and the score tiles),
+    uneven key lists, with nothing else that could differ from exact numerics:
+    one-hot projections, and inputs of 4 to 8 whose squares add exactly in any
+    order.  The caches are then the same bits.  The attention's values differ
+    by rounding, about 1e-6 of themselves, and are rounded to E4M3 twice, which
+    turns such a difference into a step for about 4e-5 of them (two boundaries
+    a step of 1/16 to 1/8); 1e-3 is the bound.  A key left out of 700 moves a
+    value by 4 percent of itself and so about half of them by a step."""
+    rng = np.random.default_rng(n + heads)
+    q_lora, out = 1024, GROUPS * O_LORA
+    shapes = {"wq_a": (q_lora, wl.HIDDEN), "wq_b": (heads * HEAD_DIM, q_lora), "wkv": (HEAD_DIM, wl.HIDDEN),
+              "wo_a": (out, heads * HEAD_DIM // GROUPS), "wo_b": (wl.HIDDEN, out)}
+    t = {k: _one_hot(ctx, rng, *v) for k, v in shapes.items()}
+    ones = {k: dev.put(np.full(k, 0x3F80, np.uint16)) for k in (q_lora, HEAD_DIM)}
+    sink = dev.put(rng.standard_normal(heads).astype(np.float32))
+    L = wohper_amd.WhMlaLayer(2, heads, NOPE, ROPE, GROUPS, O_LORA, t["wq_a"], t["wq_b"], t["wkv"], t["wo_a"], t["wo_b"],
+                              ones[q_lora], ones[HEAD_DIM], sink)
+    cap = 400
+    cache0 = rng.standard_normal((cap, HEAD_DIM)).astype(np.float32)
+    few = min(n // 2, 18)
+    positions = list(range(3, 3 + few)) + list(range(200, 200 + n - few))
+    comp = dev.put(rng.standard_normal((1000, HEAD_DIM)).astype(np.float32))
+    comps = [(comp + 4 * HEAD_DIM * int(o), int(k)) for o, k in zip(rng.integers(0, 300, n), rng.integers(1, 701, n))]
+    xs = (rng.integers(4, 9, (n, wl.HIDDEN)) * rng.choice([-1, 1], (n, wl.HIDDEN))).astype(np.float32)
+    got = {}
+    for exact in (True, False):
+        ctx.set_exact_numerics(exact)
+        got[exact] = _batch(ctx, dev, L, xs, positions, cache0, HEAD_DIM, comps)
+    assert np.array_equal(bits(got[True][1]), bits(got[False][1]))
+    a, b = got[True][0], got[False][0]
+    differ = (a != b).mean(1)
+    print(f"{heads} heads, {n} positions: share of values a step apart, most of a position {differ.max():.2e}, "
+          f"all {differ.mean():.2e}")
+    assert np.count_nonzero(a) > 0.99 * a.size and np.all(np.isfinite(b))
+    assert differ.mean() <= 1e-3 and differ.max() <= 5e-3
+    for h in t.values():
         ctx.release(h)
 
 
