@@ -695,7 +695,10 @@ int wh_mla_attention_decode_async(wh_ctx* ctx, const wh_mla_layer* layer, size_t
  * per position, then each position's window softmax over the cache rows up
  * to its own and its n_comp[i] compressed rows at comp_dev[i] (host arrays
  * of npos entries, or NULL for none).  With exact numerics the outputs
- * equal npos calls of wh_mla_attention_decode_async in position order. */
+ * equal npos calls of wh_mla_attention_decode_async in position order.  The
+ * context keeps scratch for the scores of up to 128 positions (heads x keys
+ * floats each: 67 MB for 128 of 64 heads and 2048 keys) beside the activations
+ * of all npos. */
 int wh_mla_attention_decode_batch_async(wh_ctx* ctx, const wh_mla_layer* layer, const size_t* positions, size_t npos,
                                         float* hidden_dev, float* kv_cache_dev, size_t kv_stride, size_t kv_capacity,
                                         const float* const* comp_dev, const size_t* n_comp);
@@ -753,8 +756,8 @@ int wh_hc_post_async(wh_ctx* ctx, const float* y_dev, const float* residual_dev,
  *     hidden = hc_post(z, hidden').
  * Every step is the kernel of its own entry point, so the layer is
  * bit-identical to the reference under exact numerics; with exact numerics
- * off the FP8 projections, the attention's sums, the expert matvecs and hc_pre's sums take the
- * order-free kernels (the router keeps the reference order).  Nothing is
+ * off the FP8 projections, the attention's sums, the expert matvecs and
+ * hc_pre's sums take the order-free kernels (the router keeps the reference order).  Nothing is
  * read back to the host: the whole layer can be captured (wh_graph_begin).
  * hidden_dev 16-byte aligned; the norm weights are bf16 (NULL: plain RMS
  * norm); available_dev / n_available as in wh_route_experts_async. */

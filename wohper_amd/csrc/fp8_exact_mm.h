@@ -16,7 +16,7 @@
 // Why: the vector kernel (k_fp8_gemv_multi) issues one FMA per 64 products,
 // a decoded weight's register read again for every input: 512 products of a
 // wave in the time a matrix instruction does 1024, and its LDS reads beside
-// them.  13 inputs of a layer's five projections: 103.9 -> 88.3 us,
+// them.  13 inputs of a layer's five projections: 103.9 -> 85.6 us,
 // of the 4096 x 8192 one 36.2 -> 22.2 us (6.8 us of matrix time; the rest is
 // one wave a SIMD that also decodes, stages x and waits for the barriers).
 #pragma once
